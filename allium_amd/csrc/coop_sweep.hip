@@ -173,7 +173,7 @@ __device__ __forceinline__ void assemble_row(const SweepParams &p, const CellRef
         if (interior) {
             u = gP + base + (long long)(hi ? e + p.stride[ax] : e - p.stride[ax]) * N;
             ub = hi ? 0 : P * sax;
-        } else if (refl) {
+        } else if (refl && dot < 0) {   // the table holds -1 for the directions that leave
             u = gP + ((long long)g * p.Nomega + g_refl[a * NS + s]) * p.Ndof + (long long)e * N;
             ub = hi ? P * sax : 0;
         }

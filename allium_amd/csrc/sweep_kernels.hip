@@ -193,11 +193,13 @@ __device__ __forceinline__ void cell_solve(const SweepParams &p, const int e, co
         if (inflow_known && !inflow) { wgt[s] = 0.0; continue; }
         const bool in = inflow_known ? true : (dot < 0);
         const bool refl = !interior && ((p.refl_mask >> s) & 1);
-        const bool use_nb = in && interior, use_rf = in && refl;
+        // the table holds a reflected direction for the inflow directions of a
+        // reflective side and -1 for the others: only dot < 0 may index with it
+        const bool use_nb = in && interior, use_rf = in && refl && dot < 0;
         wgt[s] = (use_nb || use_rf) ? -dot : 0.0;
         const double *nbp = p.psi + base + (long long)(hi ? e + p.stride[ax] : e - p.stride[ax]) * N;
         const double *rfp = self;
-        if (refl) rfp = p.psi + ((long long)g * p.Nomega + p.refl[a * NS + s]) * p.Ndof + (long long)e * N;
+        if (use_rf) rfp = p.psi + ((long long)g * p.Nomega + p.refl[a * NS + s]) * p.Ndof + (long long)e * N;
 #pragma unroll
         for (int m = 0; m < NF; ++m) {
             const double *addr = use_nb ? nbp + side_node<DIM, P>(s ^ 1, m) : rfp + side_node<DIM, P>(s, m);
