@@ -1259,47 +1259,65 @@ hipError_t balance_static(const SweepParams &prm, const double *psi, double *abs
 // ---------------------------------------------------------------------------
 // moments (DiscreteToMoment, src/transport_op.cpp:3-46) and block mass
 // ---------------------------------------------------------------------------
-// Four entries per thread, 256 apart: a workgroup reads 8 KB runs of each
-// direction and keeps 16 loads in flight per thread (two and eight entries
-// per thread, and one, were slower on the 64^3 S8 psi).  Each entry is summed
-// over the directions in order.
-__global__ void __launch_bounds__(256) k_moments(const double *__restrict__ psi, const double *__restrict__ omega,
-                                                 int Nomega, long long Ndof, double *__restrict__ phi)
+// phi = sum_a w_a psi_a: 8 + 8 / Nomega bytes per unknown, bound by HBM once
+// enough loads are in flight.  A thread that sums all directions of its entry
+// leaves a small phi with a few workgroups and a chain of Nomega loads each,
+// so the WV waves of a workgroup split the directions of one run of 64 E
+// entries: wave w sums its directions in order, then the waves' sums are added
+// in order through LDS (one fixed order for every launch).  psi is streamed
+// once: nontemporal loads keep it from evicting the L2 and MALL lines the next
+// sweep reuses.  us for one thread per entry / this kernel: 4096 x 40 72 / 3.1,
+// 130950 x 84 130 / 16, 262144 x 80 123 / 27, 222000 x 48 x 4 groups 99 / 52,
+// 2097152 x 80 206 / 203 (6.7 TB/s).
+template <int WV, int E, int U>
+__global__ void __launch_bounds__(64 * WV) k_moments(const double *__restrict__ psi, const double *__restrict__ omega,
+                                                     int Nomega, long long Ndof, double *__restrict__ phi)
 {
-    constexpr int E = 4;
-    const long long b = (long long)blockIdx.x * (256 * E) + threadIdx.x;
-    const long long g = blockIdx.y;
+    __shared__ double part[WV][64 * E];
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
+    const long long b = (long long)blockIdx.x * (64 * E), g = blockIdx.y;
     const double *ps = psi + g * Nomega * Ndof;
-    bool ok[E];
+    const int a0 = Nomega * w / WV, a1 = Nomega * (w + 1) / WV;
     long long i[E];
     double acc[E];
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-        i[k] = b + 256 * k;
-        ok[k] = i[k] < Ndof;
+        i[k] = b + l + 64 * k < Ndof ? b + l + 64 * k : Ndof - 1;
         acc[k] = 0.0;
     }
-#pragma unroll 4
-    for (int a = 0; a < Nomega; ++a) {
-        const double w = omega[4 * a + 3];
+#pragma unroll U
+    for (int a = a0; a < a1; ++a) {
+        const double wa = omega[4 * a + 3];
         const double *pa = ps + (long long)a * Ndof;
 #pragma unroll
-        for (int k = 0; k < E; ++k) {
-            // psi is streamed once: nontemporal loads keep it from evicting the
-            // L2 and MALL lines the next sweep reuses (281 -> 251 us at 64^3 S8)
-            const double v = __builtin_nontemporal_load(pa + (ok[k] ? i[k] : 0));
-            acc[k] = fma(w, v, acc[k]);
-        }
+        for (int k = 0; k < E; ++k) acc[k] = fma(wa, __builtin_nontemporal_load(pa + i[k]), acc[k]);
     }
 #pragma unroll
-    for (int k = 0; k < E; ++k)
-        if (ok[k]) phi[g * Ndof + i[k]] = acc[k];
+    for (int k = 0; k < E; ++k) part[w][l + 64 * k] = acc[k];
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < 64 * E && b + t < Ndof) {
+        double s = part[0][t];
+#pragma unroll
+        for (int q = 1; q < WV; ++q) s += part[q][t];
+        phi[g * Ndof + b + t] = s;
+    }
 }
 
 hipError_t launch_moments(const SweepParams &prm, const double *psi, double *phi, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_moments, dim3((unsigned)((prm.Ndof + 1023) / 1024), (unsigned)prm.G), dim3(256), 0, s, psi,
-                       prm.omega, prm.Nomega, prm.Ndof, phi);
+    // A psi that outgrows the 256 MB MALL is read from HBM: 16 waves of a
+    // workgroup on 1 KB runs reach 6.7 TB/s (203 us at 2097152 x 80, against
+    // 216 with 4 waves on 512 B).  Below, psi is partly in the MALL and more,
+    // smaller workgroups are faster: 262144 x 80 (168 MB) 27 against 36 us,
+    // 222000 x 48 x 4 (341 MB) 52 against 58.
+    const double bytes = 8.0 * prm.Ndof * prm.Nomega * prm.G;
+    if (bytes > 5e8)
+        hipLaunchKernelGGL((k_moments<16, 2, 4>), dim3((unsigned)((prm.Ndof + 127) / 128), (unsigned)prm.G),
+                           dim3(1024), 0, s, psi, prm.omega, prm.Nomega, prm.Ndof, phi);
+    else
+        hipLaunchKernelGGL((k_moments<4, 1, 8>), dim3((unsigned)((prm.Ndof + 63) / 64), (unsigned)prm.G), dim3(256),
+                           0, s, psi, prm.omega, prm.Nomega, prm.Ndof, phi);
     return hipGetLastError();
 }
 
