@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "dsa.hpp"
+#include "kernel_common.hpp"
 
 namespace allium {
 
@@ -136,29 +137,54 @@ __global__ void __launch_bounds__(kBlock) k_dg_prolong(DgLevel L, const double *
     x[t] += acc;
 }
 
-// MODE 0: x_out = x + omega dinv (b - A x); 1: out = b - A x
-template <int MODE>
+// Vertex-grid stencil.  MODE 0: out = x + omega dinv (b - A x); 1: out = b - A x;
+// 2: one sweep from zero, out = omega dinv b; 3: two sweeps from zero in one
+// pass, the neighbours' first sweep formed from their dinv and b.  The grids
+// are small (tens of thousands of vertices), so a sweep is latency: every load
+// is issued without a branch, an entry outside the grid (whose coefficient is
+// stored as zero) reads the vertex itself.  Branches around each of the 27
+// entries took 10.3 us at 24650 vertices.
+template <int MODE, int DIM>
 __global__ void __launch_bounds__(kBlock) k_st(StLevel L, const double *__restrict__ x, const double *__restrict__ b,
                                                double *__restrict__ out)
 {
-    const long long v = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (v >= L.N) return;
-    int c[3];
-    coords3(v, L.nv, c);
-    double acc = 0.0;
-    if (x) {
-        const int S = L.dim > 2 ? 27 : 9;
+    const int N = (int)L.N;
+    const int v = (int)(blockIdx.x * kBlock + threadIdx.x);
+    if (v >= N) return;
+    const double bv = b[v];
+    if constexpr (MODE == 2) {
+        out[v] = L.omega * L.dinv[v] * bv;
+    } else {
+        constexpr int S = DIM > 2 ? 27 : 9;
+        const int nx = L.nv[0], ny = L.nv[1], nxy = nx * ny;
+        const int cz = DIM > 2 ? fast_div(v, nxy, 1.0f / (float)nxy) : 0;
+        const int r = v - cz * nxy, cy = fast_div(r, nx, 1.0f / (float)nx), cx = r - cy * nx;
+        double a[S], u[S];
+#pragma unroll
         for (int k = 0; k < S; k++) {
-            const int dx = k % 3 - 1, dy = (k / 3) % 3 - 1, dz = L.dim > 2 ? k / 9 - 1 : 0;
-            const int xx = c[0] + dx, yy = c[1] + dy, zz = c[2] + dz;
-            if (xx < 0 || xx >= L.nv[0] || yy < 0 || yy >= L.nv[1] || zz < 0 || zz >= L.nv[2]) continue;
-            acc = fma(L.A[(long long)k * L.N + v], x[xx + (long long)L.nv[0] * (yy + (long long)L.nv[1] * zz)], acc);
+            const int dx = k % 3 - 1, dy = (k / 3) % 3 - 1, dz = DIM > 2 ? k / 9 - 1 : 0;
+            const bool in = cx + dx >= 0 && cx + dx < nx && cy + dy >= 0 && cy + dy < ny &&
+                            (DIM < 3 || (cz + dz >= 0 && cz + dz < L.nv[2]));
+            const int w = in ? v + dx + nx * dy + nxy * dz : v;
+            a[k] = L.A[(long long)k * N + v];
+            if constexpr (MODE == 3) u[k] = L.omega * L.dinv[w] * b[w];
+            else u[k] = x[w];
         }
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < S; k++) acc = fma(a[k], u[k], acc);
+        if constexpr (MODE == 1) out[v] = bv - acc;
+        else out[v] = u[S / 2] + L.omega * L.dinv[v] * (bv - acc);
     }
-    if constexpr (MODE == 0)
-        out[v] = (x ? x[v] : 0.0) + L.omega * L.dinv[v] * (b[v] - acc);
-    else
-        out[v] = b[v] - acc;
+}
+
+template <int MODE>
+hipError_t launch_st(const StLevel &L, const double *x, const double *b, double *out, hipStream_t s)
+{
+    const unsigned grid = (unsigned)((L.N + kBlock - 1) / kBlock);
+    if (L.dim > 2) hipLaunchKernelGGL((k_st<MODE, 3>), dim3(grid), dim3(kBlock), 0, s, L, x, b, out);
+    else hipLaunchKernelGGL((k_st<MODE, 2>), dim3(grid), dim3(kBlock), 0, s, L, x, b, out);
+    return hipGetLastError();
 }
 
 __global__ void __launch_bounds__(kBlock) k_st_restrict(StLevel F, StLevel C, const double *__restrict__ rf,
@@ -168,16 +194,19 @@ __global__ void __launch_bounds__(kBlock) k_st_restrict(StLevel F, StLevel C, co
     if (I >= C.N) return;
     int c[3];
     coords3(I, C.nv, c);
-    const int rz = F.dim > 2 ? 1 : 0, ry = F.dim > 1 ? 1 : 0;
     double acc = 0.0;
-    for (int dz = -rz; dz <= rz; dz++)
-        for (int dy = -ry; dy <= ry; dy++)
-            for (int dx = -1; dx <= 1; dx++) {
-                const int xx = 2 * c[0] + dx, yy = 2 * c[1] + dy, zz = 2 * c[2] + dz;
-                if (xx < 0 || xx >= F.nv[0] || yy < 0 || yy >= F.nv[1] || zz < 0 || zz >= F.nv[2]) continue;
-                const double w = (dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0);
-                acc = fma(w, rf[xx + (long long)F.nv[0] * (yy + (long long)F.nv[1] * zz)], acc);
-            }
+#pragma unroll
+    for (int k = 0; k < 27; k++) {
+        const int dd[3] = {k % 3 - 1, (k / 3) % 3 - 1, k / 9 - 1};
+        int f[3];
+        double w = 1.0;
+#pragma unroll
+        for (int d = 0; d < 3; d++) w *= coarse_child(F.nv[d], C.nv[d], c[d], dd[d], f[d]);
+        // a child that does not exist reads vertex 0 and is dropped
+        const long long i = w != 0.0 ? f[0] + (long long)F.nv[0] * (f[1] + (long long)F.nv[1] * f[2]) : 0;
+        const double r = rf[i];
+        acc = w != 0.0 ? fma(w, r, acc) : acc;
+    }
     rc[I] = acc;
 }
 
@@ -186,21 +215,19 @@ __global__ void __launch_bounds__(kBlock) k_st_prolong(StLevel F, StLevel C, con
 {
     const long long v = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (v >= F.N) return;
-    int c[3];
+    int c[3], lo[3], cnt[3];
     coords3(v, F.nv, c);
-    // parents per axis: even index -> one (weight 1), odd -> two (weight 1/2)
-    int lo[3], cnt[3];
-    for (int d = 0; d < 3; d++) {
-        lo[d] = c[d] >> 1;
-        cnt[d] = (c[d] & 1) ? 2 : 1;
-    }
+    for (int d = 0; d < 3; d++) cnt[d] = coarse_parents(F.nv[d], C.nv[d], c[d], lo[d]);
+    const double w = 1.0 / (cnt[0] * cnt[1] * cnt[2]);
     double acc = 0.0;
-    for (int k = 0; k < cnt[2]; k++)
-        for (int j = 0; j < cnt[1]; j++)
-            for (int i = 0; i < cnt[0]; i++) {
-                const double w = (cnt[0] == 2 ? 0.5 : 1.0) * (cnt[1] == 2 ? 0.5 : 1.0) * (cnt[2] == 2 ? 0.5 : 1.0);
-                acc = fma(w, xc[(lo[0] + i) + (long long)C.nv[0] * ((lo[1] + j) + (long long)C.nv[1] * (lo[2] + k))], acc);
-            }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int i = k & 1, j = (k >> 1) & 1, l = k >> 2;
+        const bool on = i < cnt[0] && j < cnt[1] && l < cnt[2];
+        const double u = xc[(lo[0] + (on ? i : 0)) +
+                            (long long)C.nv[0] * ((lo[1] + (on ? j : 0)) + (long long)C.nv[1] * (lo[2] + (on ? l : 0)))];
+        acc = on ? fma(w, u, acc) : acc;
+    }
     xf[v] += acc;
 }
 
@@ -308,14 +335,17 @@ hipError_t dg_prolong_add(const DgLevel &L, const double *xv, double *x, hipStre
 
 hipError_t st_jacobi(const StLevel &L, const double *x_in, const double *b, double *x_out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_st<0>, dim3(grid_of(L.N)), dim3(kBlock), 0, s, L, x_in, b, x_out);
-    return hipGetLastError();
+    return launch_st<0>(L, x_in, b, x_out, s);
+}
+
+hipError_t st_jacobi_zero(const StLevel &L, int sweeps, const double *b, double *x_out, hipStream_t s)
+{
+    return sweeps < 2 ? launch_st<2>(L, nullptr, b, x_out, s) : launch_st<3>(L, nullptr, b, x_out, s);
 }
 
 hipError_t st_resid(const StLevel &L, const double *x, const double *b, double *r, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_st<1>, dim3(grid_of(L.N)), dim3(kBlock), 0, s, L, x, b, r);
-    return hipGetLastError();
+    return launch_st<1>(L, x, b, r, s);
 }
 
 hipError_t st_restrict(const StLevel &F, const StLevel &C, const double *rf, double *rc, hipStream_t s)

@@ -34,6 +34,28 @@ struct StLevel {
     double omega;
 };
 
+// Coarsening of nv vertices on an axis to ncv: the vertices 0, 2, 4, .. and, when
+// nv is even (an odd number of elements), the last one too.  An axis with
+// ncv == nv is not coarsened.
+__host__ __device__ inline int coarse_vertices(int nv) { return nv < 3 ? nv : nv / 2 + 1; }
+// parents of fine vertex v: first coarse vertex in lo, their number (weights 1 / number)
+__host__ __device__ inline int coarse_parents(int nv, int ncv, int v, int &lo)
+{
+    const bool own = ncv == nv || !(v & 1) || v == nv - 1;
+    lo = ncv == nv ? v : (own ? (v + 1) >> 1 : v >> 1);
+    return own ? 1 : 2;
+}
+// child d in -1..1 of coarse vertex I: its fine vertex in f and the weight that
+// the vertex gives I (0: no such child)
+__host__ __device__ inline double coarse_child(int nv, int ncv, int I, int d, int &f)
+{
+    f = (ncv == nv ? I : (I == ncv - 1 ? nv - 1 : 2 * I)) + d;
+    if (d == 0) return 1.0;
+    if (ncv == nv || f < 0 || f >= nv) return 0.0;
+    int lo;
+    return coarse_parents(nv, ncv, f, lo) == 2 && (lo == I || lo + 1 == I) ? 0.5 : 0.0;
+}
+
 // x_out = x_in + omega Dinv (b - K x_in); x_in == nullptr means x_in = 0
 hipError_t dg_jacobi(const DgLevel &L, const double *x_in, const double *b, double *x_out, hipStream_t s);
 // r = b - K x
@@ -46,8 +68,10 @@ hipError_t dg_restrict(const DgLevel &L, const double *r, double *rv, hipStream_
 hipError_t dg_prolong_add(const DgLevel &L, const double *xv, double *x, hipStream_t s);
 
 hipError_t st_jacobi(const StLevel &L, const double *x_in, const double *b, double *x_out, hipStream_t s);
+// the first one or two sweeps from x = 0
+hipError_t st_jacobi_zero(const StLevel &L, int sweeps, const double *b, double *x_out, hipStream_t s);
 hipError_t st_resid(const StLevel &L, const double *x, const double *b, double *r, hipStream_t s);
-// coarse = P^T fine for the d-linear interpolation from a grid with every other vertex
+// coarse = P^T fine for the d-linear interpolation from the coarsened grid
 hipError_t st_restrict(const StLevel &F, const StLevel &C, const double *rf, double *rc, hipStream_t s);
 hipError_t st_prolong_add(const StLevel &F, const StLevel &C, const double *xc, double *xf, hipStream_t s);
 // x = Ainv b with a dense N x N inverse

@@ -81,6 +81,7 @@ constexpr int kPowerIts = 30;
 struct HostStencil {
     int dim = 0;
     int nv[3] = {1, 1, 1};
+    double h[3] = {0.0, 0.0, 0.0};   // spacing
     long long N = 0;
     std::vector<double> A;  // S x N, entry (k, v) at k * N + v
     std::vector<double> dinv;
@@ -213,6 +214,7 @@ bool galerkin_dg(const allium::Mesh &m, const allium::MipMatrix &K, HostStencil 
     L.dim = dim;
     L.N = 1;
     for (int d = 0; d < 3; d++) { L.nv[d] = d < dim ? m.nel[d] + 1 : 1; L.N *= L.nv[d]; }
+    for (int d = 0; d < dim; d++) L.h[d] = std::fabs(m.h[d]);
     L.A.assign((size_t)S * L.N, 0.0);
     double scale = 0.0;
     for (long e = 0; e < m.Ne; e++)
@@ -267,47 +269,51 @@ bool galerkin_dg(const allium::Mesh &m, const allium::MipMatrix &K, HostStencil 
     return true;
 }
 
-// Galerkin coarsening by two of a vertex grid (d-linear interpolation)
-bool coarsen(const HostStencil &F, HostStencil &C)
+// Galerkin coarsening of a vertex grid (d-linear interpolation): per axis every
+// other vertex is kept and, when the number of elements is odd, the last one
+// (allium::coarse_parents).  Point smoothing leaves the errors that are
+// rough along a widely spaced axis, so an axis waits until the closer ones
+// have been coarsened to half its spacing, unless `all`.
+bool coarsen(const HostStencil &F, bool all, HostStencil &C)
 {
     const int dim = F.dim, S = nstencil(dim);
+    double hmin = 0.0;
+    for (int d = 0; d < dim; d++)
+        if (F.nv[d] > 2 && (hmin == 0.0 || F.h[d] < hmin)) hmin = F.h[d];
     C.dim = dim;
     C.N = 1;
+    bool smaller = false;
     for (int d = 0; d < 3; d++) {
-        if (d < dim) {
-            if (F.nv[d] < 3 || (F.nv[d] - 1) % 2) return false;
-            C.nv[d] = (F.nv[d] - 1) / 2 + 1;
-        } else {
-            C.nv[d] = 1;
-        }
+        C.nv[d] = d < dim && (all || F.h[d] < 2.0 * hmin) ? allium::coarse_vertices(F.nv[d]) : F.nv[d];
+        C.h[d] = F.h[d] * (C.nv[d] < F.nv[d] ? 2.0 : 1.0);
+        smaller = smaller || C.nv[d] < F.nv[d];
         C.N *= C.nv[d];
     }
+    if (!smaller) return false;
     C.A.assign((size_t)S * C.N, 0.0);
-    const int rz = dim > 2 ? 1 : 0;
     allium::parallel_for(C.N, [&](long b, long Iend) {
         for (long I = b; I < Iend; I++) {
             const int ic[3] = {(int)(I % C.nv[0]), (int)((I / C.nv[0]) % C.nv[1]), (int)(I / ((long)C.nv[0] * C.nv[1]))};
-            for (int dz = -rz; dz <= rz; dz++)
+            for (int dz = -1; dz <= 1; dz++)
                 for (int dy = -1; dy <= 1; dy++)
                     for (int dx = -1; dx <= 1; dx++) {
-                        const int fi[3] = {2 * ic[0] + dx, 2 * ic[1] + dy, 2 * ic[2] + dz};
-                        if (fi[0] < 0 || fi[0] >= F.nv[0] || fi[1] < 0 || fi[1] >= F.nv[1] || fi[2] < 0 || fi[2] >= F.nv[2])
-                            continue;
-                        const double wI = (dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0);
+                        const int dd[3] = {dx, dy, dz};
+                        int fi[3];
+                        double wI = 1.0;
+                        for (int d = 0; d < 3; d++) wI *= allium::coarse_child(F.nv[d], C.nv[d], ic[d], dd[d], fi[d]);
+                        if (wI == 0.0) continue;
                         const long i = fi[0] + (long)F.nv[0] * (fi[1] + (long)F.nv[1] * fi[2]);
                         for (int k = 0; k < S; k++) {
                             const double a = F.A[(size_t)k * F.N + i];
                             if (a == 0.0) continue;
                             const int fj[3] = {fi[0] + k % 3 - 1, fi[1] + (k / 3) % 3 - 1, fi[2] + (dim > 2 ? k / 9 - 1 : 0)};
                             int lo[3], cnt[3];
-                            for (int d = 0; d < 3; d++) { lo[d] = fj[d] >> 1; cnt[d] = (fj[d] & 1) ? 2 : 1; }
+                            for (int d = 0; d < 3; d++) cnt[d] = allium::coarse_parents(F.nv[d], C.nv[d], fj[d], lo[d]);
+                            const double wJ = 1.0 / (cnt[0] * cnt[1] * cnt[2]);
                             for (int kz = 0; kz < cnt[2]; kz++)
                                 for (int ky = 0; ky < cnt[1]; ky++)
                                     for (int kx = 0; kx < cnt[0]; kx++) {
-                                        const int J[3] = {lo[0] + kx, lo[1] + ky, lo[2] + kz};
-                                        const double wJ = (cnt[0] == 2 ? 0.5 : 1.0) * (cnt[1] == 2 ? 0.5 : 1.0) *
-                                                          (cnt[2] == 2 ? 0.5 : 1.0);
-                                        const int o[3] = {J[0] - ic[0], J[1] - ic[1], J[2] - ic[2]};
+                                        const int o[3] = {lo[0] + kx - ic[0], lo[1] + ky - ic[1], lo[2] + kz - ic[2]};
                                         C.A[(size_t)sidx(dim, o[0], o[1], o[2]) * C.N + I] += wI * a * wJ;
                                     }
                         }
@@ -383,12 +389,14 @@ hipError_t vcycle_st(allium_dsa *d, size_t l, hipStream_t s)
     const bool last = l + 1 == d->st.size();
     if (last && d->Ainv) return allium::dense_apply(L.N, d->Ainv, d->sb[l], d->sx[l], s);
     const int nu = last ? kCoarseSweeps : std::max(1, d->desc.smooth);
-    const int total = last ? nu : 2 * nu;
-    // ping-pong so that the last sweep writes sx[l]
+    // the first two sweeps are one launch (from zero both need b only)
+    const int first = std::min(nu, 2);
+    const int total = (last ? nu : 2 * nu) - first + 1;
+    // ping-pong so that the last launch writes sx[l]
     double *cur = (total % 2) ? d->sx[l] : d->st_t[l];
     double *oth = (cur == d->sx[l]) ? d->st_t[l] : d->sx[l];
-    if ((e = allium::st_jacobi(L, nullptr, d->sb[l], cur, s)) != hipSuccess) return e;
-    for (int k = 1; k < nu; k++) {
+    if ((e = allium::st_jacobi_zero(L, first, d->sb[l], cur, s)) != hipSuccess) return e;
+    for (int k = first; k < nu; k++) {
         if ((e = allium::st_jacobi(L, cur, d->sb[l], oth, s)) != hipSuccess) return e;
         std::swap(cur, oth);
     }
@@ -797,7 +805,8 @@ int allium_dsa_create(allium_sweep_t h, const double *sigma_s, const allium_dsa_
     if (!galerkin_dg(m, K, lev[0], why)) return fail(ALLIUM_ERR_NUMERIC, why);
     while (lev.back().N > kCoarseTarget && lev.size() < 15) {
         HostStencil c;
-        if (!coarsen(lev.back(), c)) break;
+        // the level count is limited: from the ninth grid on every axis is halved
+        if (!coarsen(lev.back(), lev.size() > 8, c)) break;
         lev.push_back(std::move(c));
     }
     for (auto &L : lev) {
