@@ -1,18 +1,34 @@
-// Cooperative cell solves for local DG systems that do not fit one lane's
-// registers (3D p = 2: 27 x 27), restating src/sweep.cpp:366-475.
+// Cooperative cell solves of the 3D local DG systems whose matrices do not fit
+// one lane (p = 2: 27 x 27) or differ from element to element (p = 1: 8 x 8 on
+// general geometry), restating src/sweep.cpp:366-475.
 //
-// 16 lanes solve one cell (e, a, g), one row of a wave's DPP row each: lane t
-// assembles rows t and t + 16 (t + 16 < n) of
+// LPC lanes (8 at p = 1, 16 at p = 2) solve one cell (e, a, g): lane t holds rows
+// t and, at p = 2, t + 16 of
 //   A = sum_d Omega_d G_d + sigma M + tau Mt + sum_{outflow} (Omega.n) F
 // and of the right-hand side (source, isotropic source, upwind traces), then
 // the cell's lanes run an LU without pivoting (A + A^T is positive definite)
-// and a column-oriented back substitution.  The pivot row and each solved
-// unknown reach the other lanes of the cell by DPP row broadcast
-// (row_newbcast) from the owner lane's registers: no LDS, no synchronisation.
-// A 256-thread workgroup holds 16 cells, four per wave.
-// The launch covers one level of up to kMaxBatch independent instances, so
-// a batch of uneven meshes sweeps in max(levels) launches instead of
-// sum(levels).
+// and a column-oriented back substitution; the pivot row and each solved
+// unknown reach the other lanes by DPP row broadcast.  No LDS, no barriers.
+//
+// Assembly.  The cells of a level are ordered by element, so the 4 (p = 2) or 8
+// (p = 1) cells of a wave mostly share their element and differ in direction,
+// and column j of all their matrices is one small matrix product: directions
+// x (coefficient of each element matrix) times (element matrices) x rows.  That
+// is v_mfma_f64_4x4x4_4b: lane i + 4 b + 16 k supplies coefficient k of cell i,
+// lane r + 4 b + 16 k entry (row 4 b + r, column j) of element matrix k, and lane
+// r + 4 b + 16 i receives the sum for cell i.  One MFMA adds the three gradient
+// blocks and the mass, a second the three faces that node j lies on (weight
+// max(Omega.n, 0)), a third, with the same face operand and the weighted upwind
+// trace at node j as coefficient, the inflow part of the right-hand side.  So a
+// matrix entry is loaded once per wave and not once per cell, as columns of
+// consecutive lanes.  A wave with several elements repeats the product per
+// element with the other cells' coefficients zero.  Reading each row per cell
+// (27 doubles 216 B apart in every lane) kept the L1's return path busy 94 % of
+// the time.  Measured before / after, ms: 16^3 + 18^3 + 21^3 p = 2 S12 batch 10.7 / 8.2,
+// uniform 24^3 p = 2 S12 5.1 / 4.6, 26 x 23 x 29 p = 1 S8 (one lane per cell before)
+// 1.80 / 0.90, 48^3 p = 1 S8 8.2 / 3.2.  What is left is issue: about 2000 vector and
+// 216 matrix instructions per wave of four 27 x 27 cells at two waves per SIMD.
+#include <type_traits>
 #include <utility>
 
 #include "device.hpp"
@@ -21,30 +37,103 @@
 namespace allium {
 
 bool coop_supported(int dim, int p) { return dim == 3 && p == 2; }
+bool coop_level_supported(int dim, int p, bool uniform) { return dim == 3 && (p == 2 || (p == 1 && !uniform)); }
 
-// every entry of r is computed before any code after this point that the
-// compiler would otherwise hoist (empty asm statements keep their order)
-template <int N>
-__device__ __forceinline__ void fence_row(double (&r)[N])
-{
-#pragma unroll
-    for (int j = 0; j < N; ++j) asm volatile("" : "+v"(r[j]));
-}
+namespace {
 
-template <int First, int Count>
-struct AxisRange {
-    static constexpr int first = First, count = Count;
+template <int P>
+struct Coop {
+    static constexpr int Q = P + 1, N = Q * Q * Q, NF = Q * Q;
+    static constexpr int LPC = P == 1 ? 8 : 16;             // lanes per cell
+    static constexpr int RS = (N + LPC - 1) / LPC;          // rows per lane
+    static constexpr int CPW = 64 / LPC;                    // cells per wave
 };
 
-// lane L of each 16-lane row of the wave, to every lane of that row.  Every
-// lane is active where this is called, so the source lane is always valid and
-// bound_ctrl (zero for an invalid source) only spares the copy of an old value.
-template <int L, typename T>
-__device__ __forceinline__ T row_bcast(T x)
+// lane L of each cell's LPC lanes, to all of them.  Every lane is active where
+// this is called, so the source lane is always valid and bound_ctrl (zero for
+// an invalid source) only spares the copy of an old value.
+template <int LPC, int L, typename T>
+__device__ __forceinline__ T cell_bcast(T x)
 {
-    static_assert(L >= 0 && L < 16, "row_newbcast takes a lane of the row");
-    return __builtin_amdgcn_update_dpp((T)0, x, 0x150 + L, 0xF, 0xF, true);
+    static_assert(L >= 0 && L < LPC && (LPC == 8 || LPC == 16), "row_newbcast takes a lane of the row");
+    if constexpr (LPC == 16) {
+        return __builtin_amdgcn_update_dpp((T)0, x, 0x150 + L, 0xF, 0xF, true);
+    } else {
+        // two cells in a row of 16: banks 0, 1 take lane L, banks 2, 3 lane L + 8
+        const T lo = __builtin_amdgcn_update_dpp((T)0, x, 0x150 + L, 0xF, 0xF, true);
+        return __builtin_amdgcn_update_dpp(lo, x, 0x150 + L + 8, 0xF, 0xC, false);
+    }
 }
+
+// One LU step on W columns (RS rows a lane): each row takes n[r] times the pivot
+// row's entry, which the FMA reads from lane L of the cell by DPP.  The compiler
+// makes a 64-bit DPP move and an FMA of this; v_fmac_f64_dpp is both (788 FMAs
+// and 431 moves of a 27 x 27 solve became 756 FMAs).  A DPP operand may not be
+// read in the two instructions after the one that writes it: the s_nop covers
+// what ran before, and inside a block no instruction reads what one of the two
+// before it wrote.  Nothing here may read an MFMA result directly (the compiler
+// inserts the waits for its own instructions only): the first step is plain C++.
+// DST: rows of the other row set (never the pivot's), SELF: the pivot's row set.
+#define ALLIUM_FMAC(D, S, M, L, B) "v_fmac_f64_dpp %" #D ", %" #S ", %" #M " row_newbcast:%" #L " row_mask:0xf bank_mask:" #B "\n"
+template <int L>
+__device__ __forceinline__ void fmac_self16(double &a, double &b, double &c, double &d, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 0, 4, 5, 0xf) ALLIUM_FMAC(1, 1, 4, 5, 0xf) ALLIUM_FMAC(2, 2, 4, 5, 0xf)
+            ALLIUM_FMAC(3, 3, 4, 5, 0xf)
+        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+        : "v"(n), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fmac_self16(double &a, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 0, 1, 2, 0xf) : "+v"(a) : "v"(n), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fmac_cross16(double &a, double &b, double &c, double &d, double sa, double sb, double sc,
+                                             double sd, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 4, 8, 9, 0xf) ALLIUM_FMAC(1, 5, 8, 9, 0xf) ALLIUM_FMAC(2, 6, 8, 9, 0xf)
+            ALLIUM_FMAC(3, 7, 8, 9, 0xf)
+        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+        : "v"(sa), "v"(sb), "v"(sc), "v"(sd), "v"(n), "i"(L));
+}
+template <int L>
+__device__ __forceinline__ void fmac_cross16(double &a, double sa, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 1, 2, 3, 0xf) : "+v"(a) : "v"(sa), "v"(n), "i"(L));
+}
+// two cells in a row of 16: banks 0, 1 take lane L, banks 2, 3 lane L + 8
+template <int L>
+__device__ __forceinline__ void fmac_self8(double &a, double &b, double &c, double &d, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 0, 4, 5, 0x3) ALLIUM_FMAC(1, 1, 4, 5, 0x3) ALLIUM_FMAC(2, 2, 4, 5, 0x3)
+            ALLIUM_FMAC(3, 3, 4, 5, 0x3) ALLIUM_FMAC(0, 0, 4, 6, 0xc) ALLIUM_FMAC(1, 1, 4, 6, 0xc)
+                ALLIUM_FMAC(2, 2, 4, 6, 0xc) ALLIUM_FMAC(3, 3, 4, 6, 0xc)
+        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+        : "v"(n), "i"(L), "i"(L + 8));
+}
+template <int L>
+__device__ __forceinline__ void fmac_self8(double &a, double n)
+{
+    asm("s_nop 1\n" ALLIUM_FMAC(0, 0, 1, 2, 0x3) "s_nop 1\n" ALLIUM_FMAC(0, 0, 1, 3, 0xc)
+        : "+v"(a)
+        : "v"(n), "i"(L), "i"(L + 8));
+}
+// the value of lane L of the cell where an asm above may have written x
+template <int LPC, int L>
+__device__ __forceinline__ double cell_bcast_after(double x)
+{
+    double y;
+    if constexpr (LPC == 16)
+        asm("s_nop 1\nv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf" : "=v"(y) : "v"(x), "i"(L));
+    else
+        asm("s_nop 1\nv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0x3\n"
+            "v_mov_b64_dpp %0, %1 row_newbcast:%3 row_mask:0xf bank_mask:0xc"
+            : "=&v"(y)
+            : "v"(x), "i"(L), "i"(L + 8));
+    return y;
+}
+#undef ALLIUM_FMAC
 
 template <typename F, int... K>
 __device__ __forceinline__ void for_each_k(F &&f, std::integer_sequence<int, K...>)
@@ -52,392 +141,330 @@ __device__ __forceinline__ void for_each_k(F &&f, std::integer_sequence<int, K..
     (f(std::integral_constant<int, K>{}), ...);
 }
 
-// one cell (e, a, g) of a level and what every row of it shares
-template <int DIM, int P>
-struct CellRef {
-    int e, a, g;
-    double om[3], sig;
-    long long base, off;   // psi offsets of direction (g, a) and of the cell
-    int c[3];              // element coordinates
+// Columns J .. of one LU step with pivot K (the last column is the right-hand
+// side): M[r][j] += n[r] * (pivot row's M[K / LPC][j]).
+template <int LPC, int RS, int NC, int K, int J>
+__device__ __forceinline__ void lu_columns(double (&M)[RS][NC], const double (&n)[RS])
+{
+    constexpr int kr = K / LPC, L = K % LPC, left = NC - J;
+    if constexpr (left > 0) {
+        constexpr int W = left >= 4 ? 4 : 1;
+        constexpr bool self = LPC * kr + LPC - 1 > K, cross = kr + 1 < RS;
+        static_assert(RS <= 2, "the other row set is the next one");
+        if constexpr (cross) {
+            if constexpr (W == 4)
+                fmac_cross16<L>(M[kr + 1][J], M[kr + 1][J + 1], M[kr + 1][J + 2], M[kr + 1][J + 3], M[kr][J],
+                                M[kr][J + 1], M[kr][J + 2], M[kr][J + 3], n[kr + 1]);
+            else
+                fmac_cross16<L>(M[kr + 1][J], M[kr][J], n[kr + 1]);
+        }
+        if constexpr (self) {
+            if constexpr (LPC == 16) {
+                if constexpr (W == 4) fmac_self16<L>(M[kr][J], M[kr][J + 1], M[kr][J + 2], M[kr][J + 3], n[kr]);
+                else fmac_self16<L>(M[kr][J], n[kr]);
+            } else {
+                if constexpr (W == 4) fmac_self8<L>(M[kr][J], M[kr][J + 1], M[kr][J + 2], M[kr][J + 3], n[kr]);
+                else fmac_self8<L>(M[kr][J], n[kr]);
+            }
+        }
+        lu_columns<LPC, RS, NC, K, J + W>(M, n);
+    }
+}
+
+__device__ __forceinline__ double mfma4(double a, double b, double c)
+{
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+
+template <typename T>
+__device__ __forceinline__ T by_axis(int ax, T x, T y, T z)
+{
+    return ax == 0 ? x : (ax == 1 ? y : z);
+}
+
+// m[r][j]: the lanes (16 per axis) whose row of set r has the coordinate of node j
+// on the lane's axis
+template <int P>
+struct SideLanes {
+    unsigned long long m[Coop<P>::RS][Coop<P>::N];
 };
-
-// the cell of workgroup-local slot `slot`; valid is false past the level's end
-template <int DIM, int P>
-__device__ __forceinline__ CellRef<DIM, P> load_cell(const SweepParams &p, const CoopLevel &cl, int inst, long long wg0,
-                                                     int slot, bool &valid)
+template <int P>
+constexpr SideLanes<P> side_lanes()
 {
-    constexpr int N = Sh<DIM, P>::N;
-    CellRef<DIM, P> cr;
-    const int local = (int)(wg0 - cl.start[inst]) + slot;
-    valid = local < cl.ncells[inst] * p.G;
-    cr.e = cr.a = cr.g = 0;
-    if (valid) {
-        const int nc = cl.ncells[inst];
-        cr.g = local / nc;
-        const uint32_t cell = as_global(p.cells)[cl.cbeg[inst] + (local - cr.g * nc)];
-        cr.e = (int)(cell >> 10);
-        cr.a = (int)(cell & 1023u);
-    }
-    const auto g_omega = as_global(p.omega);
-    for (int d = 0; d < 3; ++d) cr.om[d] = g_omega[4 * cr.a + d];
-    cr.sig = as_global(p.sigma)[(long long)cr.g * p.Ne + cr.e];
-    cr.base = ((long long)cr.g * p.Nomega + cr.a) * p.Ndof;
-    cr.off = cr.base + (long long)cr.e * N;
-    cr.c[0] = cr.e % p.nel[0];
-    cr.c[1] = (cr.e / p.nel[0]) % p.nel[1];
-    cr.c[2] = cr.e / (p.nel[0] * p.nel[1]);
-    return cr;
+    using C = Coop<P>;
+    constexpr int Q = C::Q;
+    SideLanes<P> s{};
+    for (int r = 0; r < C::RS; ++r)
+        for (int j = 0; j < C::N; ++j)
+            for (int l = 0; l < 48; ++l) {
+                const int t = l % C::LPC, row = t + C::LPC * r < C::N ? t + C::LPC * r : t;
+                const int step = l / 16 == 0 ? 1 : (l / 16 == 1 ? Q : Q * Q);
+                if ((row / step) % Q == (j / step) % Q) s.m[r][j] |= 1ull << l;
+            }
+    return s;
 }
+template <int P>
+constexpr SideLanes<P> kSideLanes = side_lanes<P>();
 
-// row rr of the cell's local system into (Ar, b)
-template <int DIM, int P, bool UNI>
-__device__ __forceinline__ void assemble_row(const SweepParams &p, const CellRef<DIM, P> &cr, const int rr,
-                                             double (&Ar)[Sh<DIM, P>::N], double &b)
+// the cells of one wave: items first .. first + CPW of the instance's level
+template <int P, bool UNI, typename T>
+__device__ __forceinline__ void coop_wave(const SweepParams &p, const CoopLevel &cl, int inst, long long wg0)
 {
-    using S = Sh<DIM, P>;
-    constexpr int N = S::N, NF = S::NF, NS = S::NS, Q = P + 1;
+    using C = Coop<P>;
+    constexpr int Q = C::Q, N = C::N, NF = C::NF, LPC = C::LPC, RS = C::RS;
+    const int nc = cl.ncells[inst], items = nc * p.G;
+    const int first = (int)(wg0 - cl.start[inst]) + (int)(threadIdx.x >> 6) * C::CPW;
+    if (first >= items) return;   // wave-uniform
     // every table read through p is global memory
-    const auto g_K = as_global(p.K), g_Mu = as_global(p.Mu), g_Mt = as_global(p.Mt), g_Gd = as_global(p.Gd);
-    const auto g_src = as_global(p.src), g_iso = as_global(p.iso), g_F = as_global(p.Fface);
-    const auto g_fnor = as_global(p.fnor);
-    const auto g_refl = as_global(p.refl);
+    const auto g_cells = as_global(p.cells);
     const auto g_psi = as_global(p.psi);
-    const int e = cr.e, a = cr.a, g = cr.g;
-    const double(&om)[3] = cr.om;
-    const double sig = cr.sig;
-    const long long base = cr.base, off = cr.off;
-    const int(&c)[3] = cr.c;
-    b = 0.0;
-    if (p.src) b = g_src[off + rr];
-    if (p.iso) b += g_iso[(long long)g * p.Ndof + (long long)e * N + rr];
+    // slots past the level's end repeat its last cell and are not stored
+    auto cell_at = [&](int slot, int &e, int &a, int &g) {
+        const int it = first + slot < items ? first + slot : items - 1;
+        g = p.G > 1 ? it / nc : 0;
+        const uint32_t cell = g_cells[cl.cbeg[inst] + (it - g * nc)];
+        e = (int)(cell >> 10);
+        a = (int)(cell & 1023u);
+    };
 
-    // Faces, one axis at a time: a node lies on at most one side per axis (the
-    // low side where its coordinate on the axis is 0, the high side where it
-    // is P).  Every address follows from the cell alone, so the face normal,
-    // the face-mass row and the upwind trace are loaded without branches, and
-    // the sign of Omega.n only selects what they are added to.  The inflow
-    // traces go into b before the element matrices are read (the row sum is
-    // not live yet); on non-uniform geometry the outflow face blocks join the
-    // row after them (a uniform mesh has them in K).  Both passes take the
-    // sides in the order 2 axis + {low, high}, as one loop over the sides would.
-    const int ic[3] = {rr % Q, (rr / Q) % Q, rr / (Q * Q)};
-    // the node's side on axis ax (-1: none) and its face-lexicographic index there
-    auto side_of = [&](int ax, int &k) {
-        k = ax == 0 ? ic[1] + Q * ic[2] : (ax == 1 ? ic[0] + Q * ic[2] : ic[0] + Q * ic[1]);
-        return ic[ax] == 0 ? 2 * ax : (ic[ax] == P ? 2 * ax + 1 : -1);
-    };
-    // node l of a side of axis ax, with coordinate 0 on the axis
-    auto side_base = [](int ax, int l) {
-        return ax == 0 ? Q * (l % Q) + Q * Q * (l / Q) : (ax == 1 ? l % Q + Q * Q * (l / Q) : l);
-    };
-    // face of side s (non-uniform geometry)
-    auto face_of = [&](int s) {
-        const int ax = s >> 1;
-        int cf[3] = {c[0], c[1], c[2]};
-        cf[ax] += s & 1;
-        return p.foff[ax] + cf[0] + p.fext[ax][0] * (cf[1] + p.fext[ax][1] * cf[2]);
-    };
-    double dots[DIM];   // Omega.n on the node's side of each axis, 0 where it has none
-    auto gF = g_F;
-    auto gN = g_fnor;
-    auto gP = g_psi;
+    double A[RS][N], b[RS];
 #pragma unroll
-    for (int ax = 0; ax < DIM; ++ax) {
-        // one axis's loads in flight at a time
-        if (ax > 0) asm volatile("" : "+v"(b), "+s"(gF), "+s"(gN), "+s"(gP));
-        int k;
-        const int sd = side_of(ax, k);
-        const bool on = sd >= 0;
-        const int hi = sd & 1, s = 2 * ax + hi;
-        const bool interior = hi ? (c[ax] < p.nel[ax] - 1) : (c[ax] > 0);
-        double dot;
-        gptr<const double> F;
+    for (int r = 0; r < RS; ++r) {
+        b[r] = 0.0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) A[r][j] = 0.0;
+    }
+
+    const int lane = threadIdx.x & 63, grp = lane >> 4, half = P == 1 ? (lane >> 3) & 1 : 0, t = lane & (LPC - 1);
+    // The cell whose coefficients the lane supplies: coefficient grp of the
+    // gradients (Omega_x, Omega_y, Omega_z) and the mass (sigma), axis grp of the faces.
+    int eA, aA, gA;
+    cell_at((lane & 3) + 4 * half, eA, aA, gA);
+    // ... and the cell whose rows it holds
+    const int slot = grp + 4 * half;
+    const bool store = first + slot < items;
+    int eD, aD, gD;
+    cell_at(slot, eD, aD, gD);
+    const long long off = ((long long)gD * p.Nomega + aD) * p.Ndof + (long long)eD * N;
+    const auto g_omega = as_global(p.omega);
+    const double om[3] = {g_omega[4 * aA], g_omega[4 * aA + 1], g_omega[4 * aA + 2]};
+    const double sig = as_global(p.sigma)[(long long)gA * p.Ne + eA];
+    const int ax = grp < 3 ? grp : 0;
+    const double om_ax = by_axis(ax, om[0], om[1], om[2]);
+    const auto own = g_psi + (((long long)gA * p.Nomega + aA) * p.Ndof + (long long)eA * N);
+    const int sax = by_axis(ax, 1, Q, Q * Q);                       // node stride along the axis
+    const long long nb = (long long)by_axis(ax, p.stride[0], p.stride[1], p.stride[2]) * N;
+    // rows of the lane and their face-lexicographic index
+    int row[RS], kt[RS];
+#pragma unroll
+    for (int r = 0; r < RS; ++r) {
+        row[r] = t + LPC * r < N ? t + LPC * r : t;   // a lane without a last row repeats its first
+        const int i0 = row[r] % Q, i1 = (row[r] / Q) % Q, i2 = row[r] / (Q * Q);
+        kt[r] = by_axis(ax, i1 + Q * i2, i0 + Q * i2, i0 + Q * i1);
+    }
+
+    unsigned long long todo = ~0ull;
+    while (todo) {
+        // a uniform mesh has one element's matrices: one pass for every cell
+        const int es = UNI ? eA : __builtin_amdgcn_readlane(eA, __builtin_ctzll(todo));
+        const bool mine = UNI || eA == es;
+        todo = UNI ? 0 : todo & ~__ballot(mine);
+        const int c2 = fast_div(es, p.stride[2], p.inv_nel01), rem = es - c2 * p.stride[2];
+        const int c1 = fast_div(rem, p.nel[0], p.inv_nel0), c0 = rem - c1 * p.nel[0];
+        const int c_ax = by_axis(ax, c0, c1, c2), last = by_axis(ax, p.nel[0], p.nel[1], p.nel[2]) - 1;
+        // the element's faces normal to the lane's axis: table index of the low
+        // one and distance to the high one
+        int flo, fdh;
         if constexpr (UNI) {
-            dot = hi ? om[ax] : -om[ax];
-            F = gF + s * NF * NF + k * NF;
+            flo = 2 * ax;
+            fdh = 1;
         } else {
-            const int f = face_of(s);
-            dot = 0.0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) dot = fma(om[d], gN[3 * f + d], dot);
-            if (!hi && interior) dot = -dot;
-            F = gF + (size_t)f * NF * NF + k * NF;
+            const int f0 = p.foff[0] + c0 + p.fext[0][0] * (c1 + p.fext[0][1] * c2);
+            const int f1 = p.foff[1] + c0 + p.fext[1][0] * (c1 + p.fext[1][1] * c2);
+            const int f2 = p.foff[2] + c0 + p.fext[2][0] * (c1 + p.fext[2][1] * c2);
+            flo = by_axis(ax, f0, f1, f2);
+            fdh = by_axis(ax, 1, p.fext[1][0], p.fext[2][0] * p.fext[2][1]);
         }
-        // upwind trace: the neighbour's nodes on the opposite side, or on a
-        // reflective side the reflected direction's own nodes; elsewhere the
-        // cell's own entries stand in as an in-bounds address and are not used
-        const bool refl = !interior && ((p.refl_mask >> s) & 1);
-        const int sax = ax == 0 ? 1 : (ax == 1 ? Q : Q * Q);   // node stride along the axis
-        gptr<const double> u = gP + off;
-        int ub = 0;
-        if (interior) {
-            u = gP + base + (long long)(hi ? e + p.stride[ax] : e - p.stride[ax]) * N;
-            ub = hi ? 0 : P * sax;
-        } else if (refl && dot < 0) {   // the table holds -1 for the directions that leave
-            u = gP + ((long long)g * p.Nomega + g_refl[a * NS + s]) * p.Ndof + (long long)e * N;
-            ub = hi ? P * sax : 0;
+        // Omega.n on the low and high side
+        const bool in_lo = c_ax > 0, in_hi = c_ax < last;
+        double dlo, dhi;
+        if constexpr (UNI) {
+            dlo = -om_ax;
+            dhi = om_ax;
+        } else {
+            const auto fn = as_global(p.fnor) + 3LL * flo, fh = fn + 3LL * fdh;
+            dlo = fma(om[2], fn[2], fma(om[1], fn[1], om[0] * fn[0]));
+            dhi = fma(om[2], fh[2], fma(om[1], fh[1], om[0] * fh[0]));
+            dlo = in_lo ? -dlo : dlo;
         }
-        dots[ax] = on ? dot : 0.0;
-        double acc = 0.0;
+        dlo = mine && grp < 3 ? dlo : 0.0;
+        dhi = mine && grp < 3 ? dhi : 0.0;
+        // where the upwind trace at node j of the side is read: lo + j, hi + j; no
+        // inflow there reads zeros (at most 35 past the start, the buffer has 64)
+        const auto zero = as_global(p.zeros);
+        gptr<const double> lo = zero, hi = zero;
+        if (dlo < 0) {
+            if (in_lo) lo = own - nb + P * sax;
+            else if ((p.refl_mask >> (2 * ax)) & 1)
+                lo = g_psi + ((long long)gA * p.Nomega + as_global(p.refl)[aA * 6 + 2 * ax]) * p.Ndof + (long long)eA * N;
+        }
+        if (dhi < 0) {
+            if (in_hi) hi = own + nb - P * sax;
+            else if ((p.refl_mask >> (2 * ax + 1)) & 1)
+                hi = g_psi + ((long long)gA * p.Nomega + as_global(p.refl)[aA * 6 + 2 * ax + 1]) * p.Ndof +
+                     (long long)eA * N;
+        }
+        const double coef = mine ? (grp < 3 ? om_ax : sig) : 0.0;
+        // element matrix grp, column-major, and the face block of the lane's axis
+        // (symmetric: entry (k, l) read at l NF + k)
+        const long long ee = UNI ? 0 : es;
+        auto mat = grp < 3 ? as_global(p.Gd) + (ee * 3 + grp) * (N * N) : as_global(p.Mu) + ee * (N * N);
+        auto fb = as_global(p.Fface) + (long long)flo * (NF * NF);
+        // table offset of face node (j0, j1, j2) from (0, 0, 0): one part per axis,
+        // along the lane's axis the step to the high face
+        int fo[3][Q];
 #pragma unroll
-        for (int l = 0; l < NF; ++l) acc = fma(F[l], u[ub + side_base(ax, l)], acc);
-        const bool inflow = on && dot < 0 && (interior || refl);
-        b = inflow ? fma(-dot, acc, b) : b;
-    }
-
-    // Each matrix row is read in two halves.  The half's row pointers pass
-    // through an empty asm after fences on every entry of the running sum, so
-    // the compiler cannot hoist all the row loads ahead of the sums (all 5 N of
-    // the jittered case took 256 VGPRs + AGPRs, one wave per SIMD); halves keep
-    // the kernel at 128 VGPRs, four waves per SIMD.
-    constexpr int H = (N + 1) / 2;
-    if constexpr (UNI) {
-        auto K = g_K + ((size_t)a * N + rr) * N;   // includes tau * Mt and the outflow faces
-        auto Mu = g_Mu + (size_t)rr * N;
-        asm volatile("" : "+v"(K), "+v"(Mu), "+v"(b));
+        for (int d = 0; d < 3; ++d) {
+            const int st = d == 0 ? NF : by_axis(ax, d == 1 ? NF : Q * NF, d == 1 ? 0 : Q * NF, Q * NF);
 #pragma unroll
-        for (int j = 0; j < H; ++j) Ar[j] = fma(sig, Mu[j], K[j]);
-        fence_row<H>(reinterpret_cast<double(&)[H]>(Ar));
-        asm volatile("" : "+v"(K), "+v"(Mu));
+            for (int v = 0; v < Q; ++v) fo[d][v] = ax == d ? (v == P ? fdh * NF * NF : 0) : v * st;
+        }
+        // nodes by their coordinate on the lane's axis: 0 low side, P high side,
+        // between them neither
+        auto dv = [&](int v) { return v == 0 ? dlo : (v == P ? dhi : 0.0); };
+        auto uv = [&](int v) { return v == 0 ? lo : (v == P ? hi : zero); };
+        // Columns in node order, CH at a time: the loads of the next chunk are issued
+        // before the products of this one (NB = 2 buffers).  At p = 1 all columns fit.
+        // A p = 2 uniform mesh reads fewer lines and is faster with one column at a
+        // time and a third wave in the registers (24^3 S12: 4.5 against 5.5 ms).
+        constexpr int CH = P == 1 ? N : (UNI ? 1 : Q), NC = N / CH, NB = NC > 1 && !UNI ? 2 : 1;
+        static_assert(N % CH == 0, "whole chunks");
+        double u[NB][CH], m[NB][CH][RS], f[NB][CH][RS];
+        auto load = [&](auto cc) {
+            constexpr int c = decltype(cc)::value, v = c % NB;
+            if constexpr (c < NC) {
 #pragma unroll
-        for (int j = H; j < N; ++j) Ar[j] = fma(sig, Mu[j], K[j]);
-    } else {
-        auto Gd = g_Gd + (size_t)e * DIM * N * N + (size_t)rr * N;
-        auto Mu = g_Mu + (size_t)e * N * N + (size_t)rr * N;
-        auto Mt = g_Mt + (size_t)e * N * N + (size_t)rr * N;
-        // A steady problem (tau = 0) skips the time-mass row, whose
-        // fma(0, Mt, .) would leave the sum unchanged.
-        // (the first phase starts after the face pass: its pointer passes through
-        // the same empty asm as b)
-        auto phase = [&](auto q, double c, bool first) {
-            if (!first) fence_row<N>(Ar);
-            asm volatile("" : "+v"(q), "+v"(b));
+                for (int i = 0; i < CH; ++i) {
+                    const int j = c * CH + i, j0 = j % Q, j1 = (j / Q) % Q, j2 = j / (Q * Q);
+                    u[v][i] = by_axis(ax, uv(j0), uv(j1), uv(j2))[j];
+                    const auto fj = fb + (fo[0][j0] + fo[1][j1] + fo[2][j2]);
 #pragma unroll
-            for (int j = 0; j < H; ++j) Ar[j] = first ? c * q[j] : fma(c, q[j], Ar[j]);
-            fence_row<H>(reinterpret_cast<double(&)[H]>(Ar));
-            asm volatile("" : "+v"(q));
-#pragma unroll
-            for (int j = H; j < N; ++j) Ar[j] = first ? c * q[j] : fma(c, q[j], Ar[j]);
-        };
-        phase(Gd, om[0], true);
-#pragma unroll
-        for (int d = 1; d < DIM; ++d) phase(Gd + (size_t)d * N * N, om[d], false);
-        phase(Mu, sig, false);
-        if (p.timedep) phase(Mt, p.tau, false);
-        // outflow: the own face block joins the row (the face-mass rows were
-        // read by the face pass, so these loads are cache hits)
-        // Each row is loaded before any of it is used (a row loaded only where
-        // it is added would become one branch and one round trip per entry):
-        // the first axis's row, then the other two in one batch.
-        auto outflow_rows = [&](auto axes) {
-            fence_row<N>(Ar);
-            asm volatile("" : "+s"(gF));
-            constexpr int A0 = decltype(axes)::first, NA = decltype(axes)::count;
-            double Fk[NA][NF];
-#pragma unroll
-            for (int t = 0; t < NA; ++t) {
-                const int ax = A0 + t;
-                int k;
-                const int hi = side_of(ax, k) & 1;
-                const auto F = gF + (size_t)face_of(2 * ax + hi) * NF * NF + k * NF;
-#pragma unroll
-                for (int l = 0; l < NF; ++l) Fk[t][l] = F[l];
-            }
-#pragma unroll
-            for (int t = 0; t < NA; ++t) fence_row<NF>(Fk[t]);
-#pragma unroll
-            for (int t = 0; t < NA; ++t) {
-                const int ax = A0 + t;
-                int k;
-                const int hi = side_of(ax, k) & 1;
-                const int sax = ax == 0 ? 1 : (ax == 1 ? Q : Q * Q);
-                const bool outflow = dots[ax] > 0;
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int l = 0; l < NF; ++l) {
-                        const int j = h * P * sax + side_base(ax, l);
-                        Ar[j] = (outflow && hi == h) ? fma(dots[ax], Fk[t][l], Ar[j]) : Ar[j];
+                    for (int r = 0; r < RS; ++r) {
+                        m[v][i][r] = mat[j * N + row[r]];
+                        f[v][i][r] = fj[kt[r]];
                     }
+                }
             }
         };
-        outflow_rows(AxisRange<0, 1>{});
-        outflow_rows(AxisRange<1, DIM - 1>{});
-    }
-}
-
-// 16 lanes per cell, two rows per lane, LU by DPP row broadcast (no LDS
-// exchange): the FP64 solves and the uniform-geometry FP32 ones
-template <int DIM, int P, bool UNI, typename T>
-__device__ __forceinline__ void coop_cell_dpp(const SweepParams &p, const CoopLevel &cl, int inst, long long wg0)
-{
-    constexpr int N = Sh<DIM, P>::N;
-    static_assert(N > 16 && N <= 32, "two rows per lane of a 16-lane row");
-    const int slot = threadIdx.x >> 4, t = threadIdx.x & 15;
-    bool valid;
-    const CellRef<DIM, P> cr = load_cell<DIM, P>(p, cl, inst, wg0, slot, valid);
-    const auto g_psi = as_global(p.psi);
-    const long long off = cr.off;
-    auto assemble = [&](const int rr, double (&Ar)[N], double &b) { assemble_row<DIM, P, UNI>(p, cr, rr, Ar, b); };
-
-    // rows t and t + 16 of the cell (a lane without a second row assembles its
-    // first one again; that copy takes no part in the solve)
-    constexpr int R1 = N - 16;   // lanes with a second row
-    const int r1 = t < R1 ? t + 16 : t;
-    T A0[N], A1[N], b0, b1;
-    {
-        double Ar[N], b;
-        assemble(t, Ar, b);
-        if constexpr (sizeof(T) == 4) {
-            // FP32 rows wait in LDS (one column per thread, 27.6 KB per
-            // workgroup) while the second row is assembled: registers for
-            // more waves.  The empty asm keeps the compiler from carrying
-            // the stored values across in registers.
-            __shared__ float stash[N][256];
+        if constexpr (NB == 2) load(std::integral_constant<int, 0>{});
+        for_each_k(
+            [&](auto cc) {
+                constexpr int c = decltype(cc)::value, v = c % NB;
+                if constexpr (UNI) asm volatile("" : "+v"(mat), "+v"(fb), "+v"(lo), "+v"(hi), "+v"(b[0]));
+                load(std::integral_constant<int, c + NB - 1>{});
 #pragma unroll
-            for (int j = 0; j < N; ++j) stash[j][threadIdx.x] = (float)Ar[j];
-            b0 = (T)b;
-            asm volatile("" ::: "memory");
-            fence_row<N>(Ar);
-            assemble(r1, Ar, b);
+                for (int i = 0; i < CH; ++i) {
+                    const int j = c * CH + i;
+                    const double d = by_axis(ax, dv(j % Q), dv((j / Q) % Q), dv(j / (Q * Q)));
+                    const double out = d > 0 ? d : 0.0, inn = -d * u[v][i];
 #pragma unroll
-            for (int j = 0; j < N; ++j) A1[j] = (T)Ar[j];
-            b1 = (T)b;
-            asm volatile("" ::: "memory");
+                    for (int r = 0; r < RS; ++r) {
+                        // the row is on the same side of the lane's axis as the node
+                        const double fz =
+                            __builtin_amdgcn_inverse_ballot_w64(kSideLanes<P>.m[r][j]) ? f[v][i][r] : 0.0;
+                        b[r] = mfma4(inn, fz, b[r]);
+                        A[r][j] = mfma4(coef, m[v][i][r], mfma4(out, fz, A[r][j]));
+                    }
+                }
+            },
+            std::make_integer_sequence<int, NC>{});
+        if (p.timedep) {
+            const auto mt = as_global(p.Mt) + ee * (N * N);
+            const double tau = mine && grp == 0 ? p.tau : 0.0;
 #pragma unroll
-            for (int j = 0; j < N; ++j) A0[j] = stash[j][threadIdx.x];
-        } else {
+            for (int j = 0; j < N; ++j)
 #pragma unroll
-            for (int j = 0; j < N; ++j) A0[j] = (T)Ar[j];
-            b0 = (T)b;
-            fence_row<N>(Ar);
-            assemble(r1, Ar, b);
-#pragma unroll
-            for (int j = 0; j < N; ++j) A1[j] = (T)Ar[j];
-            b1 = (T)b;
+                for (int r = 0; r < RS; ++r) {
+                    const double v = mt[j * N + row[r]];
+                    A[r][j] = mfma4(tau, grp == 0 ? v : 0.0, A[r][j]);
+                }
         }
+    }
+#pragma unroll
+    for (int r = 0; r < RS; ++r) {
+        if (p.src) b[r] += as_global(p.src)[off + row[r]];
+        if (p.iso) b[r] += as_global(p.iso)[(long long)gD * p.Ndof + (long long)eD * N + row[r]];
     }
 
     // ---- LU without pivoting ------------------------------------------------
-    // Pivot row k is row (k & 15) of slot k >> 4 on lane k & 15.  Every lane
-    // runs every update; a row at or above the pivot takes multiplier 0.
+    // Pivot row k is row set k / LPC of lane k % LPC.  Every lane runs every
+    // update; a row at or above the pivot takes multiplier 0.
+    // Rows past the last one follow along and are never a pivot.
+    constexpr bool kAsm = sizeof(T) == 8;
+    T M[RS][N + 1], ninv[RS];   // ninv: minus the reciprocal of the row's own pivot
+#pragma unroll
+    for (int r = 0; r < RS; ++r) {
+        ninv[r] = (T)0;
+        M[r][N] = (T)b[r];
+#pragma unroll
+        for (int j = 0; j < N; ++j) M[r][j] = (T)A[r][j];
+    }
     for_each_k(
         [&](auto kc) {
-            constexpr int k = decltype(kc)::value, kl = k & 15;
-            const T piv = k < 16 ? row_bcast<kl>(A0[k]) : row_bcast<kl>(A1[k]);
+            constexpr int k = decltype(kc)::value, kr = k / LPC, kl = k % LPC;
+            T piv;
+            if constexpr (kAsm && k > 0) piv = cell_bcast_after<LPC, kl>(M[kr][k]);
+            else piv = cell_bcast<LPC, kl>(M[kr][k]);
             const T rp = fast_rcp(piv);
-            T l0 = (T)0, l1 = (T)0;
-            if constexpr (k < 15) l0 = t > k ? A0[k] * rp : (T)0;
-            l1 = (t < R1 && t + 16 > k) ? A1[k] * rp : (T)0;
+            ninv[kr] = t == kl ? -rp : ninv[kr];
+            T n[RS];
 #pragma unroll
-            for (int j = k + 1; j < N; ++j) {
-                const T pj = k < 16 ? row_bcast<kl>(A0[j]) : row_bcast<kl>(A1[j]);
-                if constexpr (k < 15) A0[j] = fma(-l0, pj, A0[j]);
-                A1[j] = fma(-l1, pj, A1[j]);
+            for (int r = 0; r < RS; ++r) {
+                n[r] = (T)0;
+                if (r >= kr) n[r] = -(M[r][k] * rp);
+                if (r == kr) n[r] = t > kl ? n[r] : (T)0;
             }
-            const T pb = k < 16 ? row_bcast<kl>(b0) : row_bcast<kl>(b1);
-            if constexpr (k < 15) b0 = fma(-l0, pb, b0);
-            b1 = fma(-l1, pb, b1);
+            if constexpr (kAsm && k > 0) {
+                lu_columns<LPC, RS, N + 1, k, k + 1>(M, n);
+            } else {
+#pragma unroll
+                for (int j = k + 1; j <= N; ++j) {
+                    const T pj = cell_bcast<LPC, kl>(M[kr][j]);
+#pragma unroll
+                    for (int r = 0; r < RS; ++r)
+                        if (LPC * r + LPC - 1 > k) M[r][j] = fma(n[r], pj, M[r][j]);
+                }
+            }
         },
         std::make_integer_sequence<int, N>{});
 
-    // ---- back substitution, one unknown per step ----------------------------
-    T x0 = (T)0, x1 = (T)0;
+    // ---- back substitution, one unknown per step: the rows above k take -U(., k) x_k
     for_each_k(
         [&](auto kc) {
-            constexpr int k = N - 1 - decltype(kc)::value, kl = k & 15;
-            const T own = k < 16 ? b0 * fast_rcp(A0[k]) : b1 * fast_rcp(A1[k]);
-            const T xk = row_bcast<kl>(own);
-            if constexpr (k < 16) x0 = t == kl ? xk : x0;
-            else x1 = t == kl ? xk : x1;
-            b0 = t < k ? fma(-A0[k], xk, b0) : b0;
-            b1 = (t < R1 && t + 16 < k) ? fma(-A1[k], xk, b1) : b1;
+            constexpr int k = N - 1 - decltype(kc)::value, kr = k / LPC, kl = k % LPC;
+            const T nown = M[kr][N] * ninv[kr];   // -x_k on its lane
+#pragma unroll
+            for (int r = 0; r <= kr; ++r) {
+                const T c = r < kr || t < kl ? M[r][k] : (T)0;
+                if constexpr (kAsm && LPC == 16) fmac_cross16<kl>(M[r][N], nown, c);
+                else if constexpr (kAsm) M[r][N] = fma(cell_bcast_after<LPC, kl>(nown), c, M[r][N]);
+                else M[r][N] = fma(cell_bcast<LPC, kl>(nown), c, M[r][N]);
+            }
         },
         std::make_integer_sequence<int, N>{});
-    if (valid) {
-        g_psi[off + t] = (double)x0;
-        if (t < R1) g_psi[off + t + 16] = (double)x1;
+    if (store) {
+#pragma unroll
+        for (int r = 0; r < RS; ++r)
+            if (t + LPC * r < N) g_psi[off + t + LPC * r] = (double)-(M[r][N] * ninv[r]);
     }
-}
-
-// 32 lanes per cell, one row per lane, the pivot row published through LDS:
-// the non-uniform FP32 solves, whose limit is the memory pipeline rather than
-// the LDS, and which keep four waves per SIMD this way
-template <int DIM, int P, bool UNI, typename T>
-__device__ __forceinline__ void coop_cell_lds(const SweepParams &p, const CoopLevel &cl, int inst, long long wg0)
-{
-    constexpr int N = Sh<DIM, P>::N;
-    static_assert(N <= 32, "one row per lane of a 32-lane group");
-    __shared__ T piv[8][N + 1];
-    const int slot = threadIdx.x >> 5, r = threadIdx.x & 31;
-    bool valid;
-    const CellRef<DIM, P> cr = load_cell<DIM, P>(p, cl, inst, wg0, slot, valid);
-    const bool row = valid && r < N;
-    const int rr = r < N ? r : 0;
-    double Ar[N], b;
-    assemble_row<DIM, P, UNI>(p, cr, rr, Ar, b);
-    // lanes without a row carry an identity row so that nothing is singular
-    T A[N], bb = (T)b;
-#pragma unroll
-    for (int j = 0; j < N; ++j) A[j] = row ? (T)Ar[j] : (T)(j == r ? 1.0 : 0.0);
-    if (!row) bb = (T)0;
-    // LU without pivoting across the cell's lanes: the owner of pivot row k
-    // publishes it through LDS; the 32 lanes of a cell are half of one wave
-    // and its pivot row is LDS no other cell touches, so the exchange needs
-    // no workgroup barrier (LDS executes a wave's instructions in order, and
-    // the wavefront-scope fences keep the compiler from moving the reads
-    // above the owner lane's write)
-    auto cell_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        if (r == k) {
-#pragma unroll
-            for (int j = k; j < N; ++j) piv[slot][j] = A[j];
-            piv[slot][N] = bb;
-        }
-        cell_sync();
-        if (r > k && r < N) {
-            const T l = A[k] * fast_rcp(piv[slot][k]);
-#pragma unroll
-            for (int j = k + 1; j < N; ++j) A[j] = fma(-l, piv[slot][j], A[j]);
-            bb = fma(-l, piv[slot][N], bb);
-        }
-        cell_sync();
-    }
-    // back substitution, one unknown per step
-    T x = (T)0;
-#pragma unroll
-    for (int k = N - 1; k >= 0; --k) {
-        if (r == k) {
-            x = bb * fast_rcp(A[k]);
-            piv[slot][0] = x;
-        }
-        cell_sync();
-        const T xk = piv[slot][0];
-        if (r < k) bb = fma(-A[k], xk, bb);
-        cell_sync();
-    }
-    if (row) as_global(p.psi)[cr.off + rr] = (double)x;
 }
 
 // BATCH: the instances' parameters are the device array prms (a level of
 // several instances); otherwise p0, one instance.  The two are separate
 // instantiations so that the parameters' address space is known (a pointer
 // selected between the two would be generic and its loads flat).
-// Layout per instantiation: the DPP cells (16 per workgroup) except for
-// non-uniform FP32 solves, which keep the LDS exchange (8 cells per workgroup).
-template <bool UNI, typename T>
-constexpr bool kCoopDpp = UNI || sizeof(T) == 8;
-template <bool UNI, typename T>
-constexpr int kCoopCellsPerGroup = kCoopDpp<UNI, T> ? 16 : 8;
-static_assert(kCoopCells % 16 == 0, "instances start on a workgroup of either layout");
-
-template <int DIM, int P, bool UNI, typename T, bool BATCH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3)))
+template <int P, bool UNI, typename T, bool BATCH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P == 1 ? 4 : (UNI ? 3 : 2))))
 k_sweep_coop(SweepParams p0, const SweepParams *__restrict__ prms, CoopLevel cl)
 {
     // Workgroups go to the 8 XCDs round robin (blockIdx.x % 8).  Each XCD takes
@@ -448,52 +475,54 @@ k_sweep_coop(SweepParams p0, const SweepParams *__restrict__ prms, CoopLevel cl)
     const long long wg = (long long)x * per + (x < rem ? x : rem) + q;
     // each instance's items start on a multiple of kCoopCells, so the instance (and
     // with it every parameter read through p) is uniform over the workgroup
-    const long long wg0 = wg * kCoopCellsPerGroup<UNI, T>;
+    const long long wg0 = wg * (4 * Coop<P>::CPW);
     int inst = 0;
     while (inst + 1 < cl.ninst && wg0 >= cl.start[inst + 1]) ++inst;
-    if constexpr (kCoopDpp<UNI, T>) {
-        if constexpr (BATCH)
-            coop_cell_dpp<DIM, P, UNI, T>(*(const SweepParams *)as_global(prms + inst), cl, inst, wg0);
-        else
-            coop_cell_dpp<DIM, P, UNI, T>(p0, cl, inst, wg0);
-    } else {
-        if constexpr (BATCH)
-            coop_cell_lds<DIM, P, UNI, T>(*(const SweepParams *)as_global(prms + inst), cl, inst, wg0);
-        else
-            coop_cell_lds<DIM, P, UNI, T>(p0, cl, inst, wg0);
-    }
+    if constexpr (BATCH)
+        coop_wave<P, UNI, T>(*(const SweepParams *)as_global(prms + inst), cl, inst, wg0);
+    else
+        coop_wave<P, UNI, T>(p0, cl, inst, wg0);
 }
 
-template <int DIM, int P, bool UNI>
-static hipError_t launch_dp(const SweepParams &p0, const SweepParams *d_prms, const CoopLevel &cl, int precision,
-                            hipStream_t s)
+template <int P, bool UNI>
+hipError_t launch_pu(const SweepParams &p0, const SweepParams *d_prms, const CoopLevel &cl, int precision, hipStream_t s)
 {
     const long long items = cl.start[cl.ninst];
     if (items <= 0) return hipSuccess;
-    auto grid_of = [items](int cells) { return (int)((items + cells - 1) / cells); };
-    if (precision == 1) {
-        const int grid = grid_of(kCoopCellsPerGroup<UNI, float>);
-        if (d_prms)
-            hipLaunchKernelGGL((k_sweep_coop<DIM, P, UNI, float, true>), dim3(grid), dim3(256), 0, s, p0, d_prms, cl);
-        else
-            hipLaunchKernelGGL((k_sweep_coop<DIM, P, UNI, float, false>), dim3(grid), dim3(256), 0, s, p0, d_prms, cl);
-    } else {
-        const int grid = grid_of(kCoopCellsPerGroup<UNI, double>);
-        if (d_prms)
-            hipLaunchKernelGGL((k_sweep_coop<DIM, P, UNI, double, true>), dim3(grid), dim3(256), 0, s, p0, d_prms, cl);
-        else
-            hipLaunchKernelGGL((k_sweep_coop<DIM, P, UNI, double, false>), dim3(grid), dim3(256), 0, s, p0, d_prms, cl);
+    constexpr int per = 4 * Coop<P>::CPW;
+    static_assert(P != 2 || per == kCoopCells, "instances start on a workgroup");
+    const dim3 grid((unsigned)((items + per - 1) / per)), block(256);
+    // FP32 solves of uniform p = 2 cells save nothing (24^3 S12: 4.72 ms against 4.57
+    // in FP64): they are the FP64 ones
+    constexpr bool f32 = !(P == 2 && UNI);
+    using F = std::conditional_t<f32, float, double>;
+    if constexpr (P == 2) {
+        if (d_prms) {
+            if (precision == 1 && f32)
+                hipLaunchKernelGGL((k_sweep_coop<P, UNI, F, true>), grid, block, 0, s, p0, d_prms, cl);
+            else
+                hipLaunchKernelGGL((k_sweep_coop<P, UNI, double, true>), grid, block, 0, s, p0, d_prms, cl);
+            return hipGetLastError();
+        }
+    } else if (d_prms) {
+        return hipErrorInvalidValue;   // batches are p = 2
     }
+    if (precision == 1 && f32)
+        hipLaunchKernelGGL((k_sweep_coop<P, UNI, F, false>), grid, block, 0, s, p0, d_prms, cl);
+    else
+        hipLaunchKernelGGL((k_sweep_coop<P, UNI, double, false>), grid, block, 0, s, p0, d_prms, cl);
     return hipGetLastError();
 }
+
+}  // namespace
 
 hipError_t launch_coop_level(const SweepParams &p0, const SweepParams *d_prms, const CoopLevel &cl, int dim, int p,
                              bool uniform, int precision, hipStream_t s)
 {
-    if (dim == 3 && p == 2)
-        return uniform ? launch_dp<3, 2, true>(p0, d_prms, cl, precision, s)
-                       : launch_dp<3, 2, false>(p0, d_prms, cl, precision, s);
-    return hipErrorInvalidValue;
+    if (!coop_level_supported(dim, p, uniform)) return hipErrorInvalidValue;
+    if (p == 1) return launch_pu<1, false>(p0, d_prms, cl, precision, s);
+    return uniform ? launch_pu<2, true>(p0, d_prms, cl, precision, s)
+                   : launch_pu<2, false>(p0, d_prms, cl, precision, s);
 }
 
 }  // namespace allium

@@ -26,7 +26,9 @@ struct SweepParams {
     const float *Muf;
     const double *Mt;       // time mass (= MassIntegrator rule matrix)
     const float *Mtf;
-    const double *Gd;       // general: Ne x dim x n x n
+    // gradient blocks, each column-major (entry (i, j) at j n + i): general Ne x dim x
+    // n x n; uniform one element's where the cooperative kernel runs
+    const double *Gd;
     const double *Fface;    // uniform: 2dim x nf x nf; general: Nf x nf x nf
     const float *Ffacef;
     const double *fnor;     // general: Nf x 3
@@ -131,6 +133,7 @@ struct DeviceSweep {
     std::vector<void *> owned;
     double *d_omega = nullptr;
     uint32_t *d_cells = nullptr;
+    uint32_t *d_ecells = nullptr;    // the cells of each level ordered by element, then direction
     uint32_t *d_wcells = nullptr;
     long long *d_cls_ptr = nullptr;  // nlevels x Nomega + 1: start of each (level, direction) class
     bool angle_independent = true;
@@ -171,10 +174,10 @@ bool fixup_supported(int dim, int p);
 hipError_t launch_sweep(DeviceSweep &ds, const double *src, const double *iso, double *psi,
                         hipStream_t stream, double *phi = nullptr);
 
-// Cooperative cell solves (local systems too large for one lane: 3D p = 2):
-// 16 lanes per cell, lane t owns rows t and t + 16, kCoopCells cells per
-// workgroup.  One launch runs one level of up to kMaxBatch independent
-// instances (batched sweeps of uneven meshes).
+// Cooperative cell solves (coop_sweep.hip): 3D p = 2, and 3D p = 1 on general
+// geometry, several lanes per cell, kCoopCells p = 2 cells per workgroup.  One
+// launch runs one level of up to kMaxBatch independent p = 2 instances (batched
+// sweeps of uneven meshes).  The cells of a level are ordered by element.
 constexpr int kMaxBatch = 16;
 constexpr int kCoopCells = 16;
 struct CoopLevel {
@@ -183,7 +186,8 @@ struct CoopLevel {
     long long cbeg[kMaxBatch];   // first cell of the level in each instance's cells array
     int ncells[kMaxBatch];       // cells of the level in each instance
 };
-bool coop_supported(int dim, int p);
+bool coop_supported(int dim, int p);   // every launch of these handles is cooperative
+bool coop_level_supported(int dim, int p, bool uniform);
 // d_prms: device array of the instances' parameters, or null with ninst == 1 to use p0
 hipError_t launch_coop_level(const SweepParams &p0, const SweepParams *d_prms, const CoopLevel &cl, int dim,
                              int p, bool uniform, int precision, hipStream_t s);

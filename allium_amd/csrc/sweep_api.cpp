@@ -159,8 +159,18 @@ int upload_all(allium_sweep *h)
         auto kf = tofloat(h->Kst);
         HIP_TRY(upload(ds.owned, &fK, kf.data(), kf.size()));
     } else {
-        HIP_TRY(upload(ds.owned, &dGd, ed.Gd.data(), ed.Gd.size()));
         HIP_TRY(upload(ds.owned, &dN, m.f_nor.data(), m.f_nor.size()));
+    }
+    if (!m.uniform || allium::coop_supported(dim, ed.p)) {
+        // column-major blocks: consecutive lanes of a cell hold consecutive rows
+        std::vector<double> gt(ed.Gd.size());
+        const size_t nn = (size_t)n * n;
+        allium::parallel_for((long)(gt.size() / nn), [&](long b0, long b1) {
+            for (size_t k = (size_t)b0 * nn; k < (size_t)b1 * nn; k += nn)
+                for (int i = 0; i < n; i++)
+                    for (int j = 0; j < n; j++) gt[k + (size_t)j * n + i] = ed.Gd[k + (size_t)i * n + j];
+        });
+        HIP_TRY(upload(ds.owned, &dGd, gt.data(), gt.size()));
     }
     HIP_TRY(upload(ds.owned, &dMu, ed.Mu.data(), ed.Mu.size()));
     HIP_TRY(upload(ds.owned, &dMm, ed.Mm.data(), ed.Mm.size()));
@@ -181,17 +191,18 @@ int upload_all(allium_sweep *h)
         HIP_TRY(upload(ds.owned, &dz, z.data(), z.size()));
         prm.zeros = dz;
     }
-    if (allium::coop_supported(dim, ed.p)) {
-        // cooperative solves read their element's matrices row by row: order
-        // each level by element, then direction, so that the cells one
-        // workgroup solves mostly share an element (cache reuse)
-        std::vector<uint32_t> cells = h->plan.cells;
-        for (int L = 0; L < h->plan.nlevels; L++)
-            std::sort(cells.begin() + h->plan.level_ptr[L], cells.begin() + h->plan.level_ptr[L + 1]);
-        HIP_TRY(upload(ds.owned, &ds.d_cells, cells.data(), cells.size()));
-    } else {
-        HIP_TRY(upload(ds.owned, &ds.d_cells, h->plan.cells.data(), h->plan.cells.size()));
+    if (allium::coop_level_supported(dim, ed.p, m.uniform)) {
+        // cooperative solves take the cells of a level ordered by element, then
+        // direction: the cells one wave solves mostly share an element
+        std::vector<uint32_t> cells(h->plan.cells.size());
+        std::vector<long> pos(h->plan.level_ptr.begin(), h->plan.level_ptr.end());
+        for (int e = 0; e < m.Ne; e++)
+            for (int a = 0; a < No; a++)
+                cells[pos[h->plan.level[(size_t)e * No + a]]++] = ((uint32_t)e << 10) | (uint32_t)a;
+        HIP_TRY(upload(ds.owned, &ds.d_ecells, cells.data(), cells.size()));
     }
+    if (allium::coop_supported(dim, ed.p)) ds.d_cells = ds.d_ecells;
+    else HIP_TRY(upload(ds.owned, &ds.d_cells, h->plan.cells.data(), h->plan.cells.size()));
     prm.cells = ds.d_cells;
     prm.refl_mask = 0;
     for (int s = 0; s < 2 * dim; s++)

@@ -248,9 +248,9 @@ __device__ __forceinline__ void cell_solve(const SweepParams &p, const int e, co
         for (int i = 0; i < N; ++i)
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                double v = om[0] * Gd[i * N + j];
+                double v = om[0] * Gd[j * N + i];
 #pragma unroll
-                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[(d * N + i) * N + j], v);
+                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[(d * N + j) * N + i], v);
                 v = fma(sig, Mu[i * N + j], v);
                 v = fma(tau, Mt[i * N + j], v);
                 A[i][j] = (T)v;
@@ -399,10 +399,10 @@ __device__ __forceinline__ void group_cell_solve(const SweepParams &p, const int
         for (int j = 0; j < RPL; ++j)
 #pragma unroll
             for (int cc = 0; cc < N; ++cc) {
-                const int ij = (r0 + j) * N + cc;
-                double v = om[0] * Gd[ij];
+                const int ij = (r0 + j) * N + cc, ji = cc * N + r0 + j;
+                double v = om[0] * Gd[ji];
 #pragma unroll
-                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[d * N * N + ij], v);
+                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[d * N * N + ji], v);
                 v = fma(sig, Mu[ij], v);
                 if (p.timedep) v = fma(p.tau, Mt[ij], v);
                 A[j][cc] = (T)v;
@@ -707,10 +707,11 @@ bool sweep_supported(int dim, int p, std::string &why)
     return false;
 }
 
-// levels of one instance through the cooperative kernel (3D p = 2)
-static hipError_t run_coop(DeviceSweep &ds, const SweepParams &prm, hipStream_t s, int mode)
+// levels of one instance through the cooperative kernel
+static hipError_t run_coop(DeviceSweep &ds, SweepParams prm, hipStream_t s, int mode)
 {
     if (mode != 0) return hipErrorInvalidValue;
+    prm.cells = ds.d_ecells;
     for (int L = 0; L < ds.nlevels; ++L) {
         CoopLevel cl{};
         cl.ninst = 1;
@@ -809,7 +810,10 @@ static hipError_t run_mode(DeviceSweep &ds, const SweepParams &prm, hipStream_t 
 {
     if (mode == 3) return run_directions<DIM, P, UNI, T>(ds, prm, stream);
     if (mode == 2) return run_persistent<DIM, P, UNI, T>(ds, prm, stream);
-    return run_levels<DIM, P, UNI, T>(ds, prm, stream);
+    // 3D p = 1 on general geometry: cooperative cells whatever ds.lanes (26 x 23 x 29
+    // S8: 0.77 ms against 1.68 with the best of 1, 2 and 4 lanes of own rows)
+    if constexpr (DIM == 3 && P == 1 && !UNI) return run_coop(ds, prm, stream, mode);
+    else return run_levels<DIM, P, UNI, T>(ds, prm, stream);
 }
 
 template <int DIM, int P>
@@ -958,25 +962,32 @@ __global__ void __launch_bounds__(256) k_apply_L(SweepParams p, const double *__
     double xl[N], yl[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) xl[i] = xe[i];
+    if constexpr (UNI) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        double acc = 0.0;
+        for (int i = 0; i < N; ++i) {
+            double acc = 0.0;
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            double v;
-            if constexpr (UNI) {
-                v = fma(sig, p.Mu[i * N + j], p.K[((size_t)a * N + i) * N + j]);   // K includes tau * Mt
-            } else {
-                const double *Gd = p.Gd + (size_t)e * DIM * N * N;
-                v = om[0] * Gd[i * N + j];
-#pragma unroll
-                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[(d * N + i) * N + j], v);
-                v = fma(sig, p.Mu[(size_t)e * N * N + i * N + j], v);
-                if (p.timedep) v = fma(p.tau, p.Mt[(size_t)e * N * N + i * N + j], v);
-            }
-            acc = fma(v, xl[j], acc);
+            for (int j = 0; j < N; ++j)   // K includes tau * Mt
+                acc = fma(fma(sig, p.Mu[i * N + j], p.K[((size_t)a * N + i) * N + j]), xl[j], acc);
+            yl[i] = acc;
         }
-        yl[i] = acc;
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) yl[i] = 0.0;
+        // column by column, as the gradient blocks are stored (the masses are symmetric)
+        const double *Gd = p.Gd + (size_t)e * DIM * N * N, *Mu = p.Mu + (size_t)e * N * N;
+        const double *Mt = p.Mt + (size_t)e * N * N;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                double v = om[0] * Gd[j * N + i];
+#pragma unroll
+                for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[(d * N + j) * N + i], v);
+                v = fma(sig, Mu[j * N + i], v);
+                if (p.timedep) v = fma(p.tau, Mt[j * N + i], v);
+                yl[i] = fma(v, xl[j], yl[i]);
+            }
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
