@@ -137,6 +137,8 @@ struct DeviceSweep {
     uint32_t *d_wcells = nullptr;
     long long *d_cls_ptr = nullptr;  // nlevels x Nomega + 1: start of each (level, direction) class
     bool angle_independent = true;
+    bool lumped = false;         // element matrices on the vertex rule
+    double h2[2] = {0.0, 0.0};   // element lengths of a uniform mesh (x, y)
     std::vector<long> wlevel_base;
     std::vector<int> wpb;
     int nparts = 1;
@@ -195,6 +197,10 @@ hipError_t reset_persistent(DeviceSweep &ds, hipStream_t stream);
 // one sweep as box-level launches (modes 4/5); the box plan must be built
 hipError_t launch_box_sweep(const DeviceSweep &ds, const SweepParams &prm, hipStream_t stream);
 bool box_sweep_supported(int dim, int p);
+// direction sweeps by rows of elements (2D uniform p = 1, 2): workgroup size, 0 where they
+// do not apply (or a strip's traces exceed the LDS)
+int row_sweep_block(const DeviceSweep &ds);
+hipError_t launch_row_sweep(const DeviceSweep &ds, const SweepParams &prm, hipStream_t stream);
 // entry (i, j) of the unit-volume tensor-product mass the box kernel uses
 double host_unit_mass(int dim, int p, int i, int j);
 bool sweep_supported(int dim, int p, std::string &why);
