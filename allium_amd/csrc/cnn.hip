@@ -63,29 +63,40 @@ constexpr int kMaxDil = 8;
 // 10 x 10 x 10 halo is loaded into LDS once, so each input voxel feeds its 27
 // taps from LDS instead of 27 cache reads.  Each output element accumulates
 // its K steps (tap-major, then 8-channel chunks) in order.
+//
+// Tiles are 8 x 8 x 8 voxels on eight waves, or 4 x 4 x 4 on one wave where a
+// sub-grid is too narrow to fill the large one.
 constexpr int kConvMT = 4;
-constexpr int kTX = 8, kTY = 8, kTZ = 8, kHX = kTX + 2, kHY = kTY + 2, kHZ = kTZ + 2;
-constexpr int kHalo = kHX * kHY * kHZ;
+template <int TE>
+struct Tile {
+    static constexpr int E = TE, H = TE + 2, halo = H * H * H, waves = TE * TE * TE / (16 * kConvMT);
+    // voxel of row v of a wave's operand tile t: (i, j, k) in the tile
+    static __device__ __forceinline__ void voxel(int w, int t, int v, int &i, int &j, int &k)
+    {
+        if constexpr (TE == 8) { i = v & 7; j = 2 * t + (v >> 3); k = w; }
+        else { i = v & 3; j = v >> 2; k = t; }
+    }
+};
 
 struct TileGeo {
     int nsx, nsy, nsz;   // sub-grid extents (the largest, at offset 0)
     int ntx, nty, ntz;   // tiles per sub-grid axis
 };
 
-__host__ __device__ inline TileGeo tile_geo(const Geo &g)
+__host__ __device__ inline TileGeo tile_geo(const Geo &g, int e)
 {
     TileGeo t;
     t.nsx = (g.nx + g.dil - 1) / g.dil;
     t.nsy = (g.ny + g.dil - 1) / g.dil;
     t.nsz = (g.nz + g.dil - 1) / g.dil;
-    t.ntx = (t.nsx + kTX - 1) / kTX;
-    t.nty = (t.nsy + kTY - 1) / kTY;
-    t.ntz = (t.nsz + kTZ - 1) / kTZ;
+    t.ntx = (t.nsx + e - 1) / e;
+    t.nty = (t.nsy + e - 1) / e;
+    t.ntz = (t.nsz + e - 1) / e;
     return t;
 }
 
-template <int CIP, int COP, int MODE>
-__global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ in, const bf16 *__restrict__ W,
+template <int CIP, int COP, int MODE, int TE>
+__global__ void __launch_bounds__(64 * Tile<TE>::waves) k_conv_t(Geo g, const bf16 *__restrict__ in, const bf16 *__restrict__ W,
                                                 const float *__restrict__ bias, bf16 *__restrict__ out_bf,
                                                 float *__restrict__ out_f, const bf16 *__restrict__ mask)
 {
@@ -94,10 +105,11 @@ __global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ 
     // voxel stride in LDS: the channels, unpadded (timed against 16, 32 and 48
     // bytes of padding per voxel, which were 28 % slower in a 64^3 inference)
     constexpr int VS = CIP * 2;
-    static_assert(MT * 16 * 8 == kTX * kTY * kTZ, "a workgroup's voxels are one tile");
+    using TL = Tile<TE>;
+    static_assert(MT * 16 * TL::waves == TE * TE * TE, "a workgroup's voxels are one tile");
     extern __shared__ __align__(16) unsigned char halo[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, grp = lane >> 4;
-    const TileGeo tg = tile_geo(g);
+    const TileGeo tg = tile_geo(g, TE);
     // workgroup -> (batch, sub-grid offset, tile)
     long long q = blockIdx.x;
     const int tx = (int)(q % tg.ntx); q /= tg.ntx;
@@ -110,10 +122,10 @@ __global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ 
     const long long b = q;
     const long long plane = (long long)g.nx * g.ny, vol = plane * g.nz;
     // halo: CH 16-byte chunks per voxel, zeros outside the grid
-    for (int c = threadIdx.x; c < kHalo * CH; c += 512) {
+    for (int c = threadIdx.x; c < TL::halo * CH; c += 64 * TL::waves) {
         const int hv = c / CH, part = c - hv * CH;
-        const int hx = hv % kHX, hy = (hv / kHX) % kHY, hz = hv / (kHX * kHY);
-        const int x = sx + d * (tx * kTX + hx - 1), y = sy + d * (ty * kTY + hy - 1), z = sz + d * (tz * kTZ + hz - 1);
+        const int hx = hv % TL::H, hy = (hv / TL::H) % TL::H, hz = hv / (TL::H * TL::H);
+        const int x = sx + d * (tx * TE + hx - 1), y = sy + d * (ty * TE + hy - 1), z = sz + d * (tz * TE + hz - 1);
         const bool ok = x >= 0 && x < g.nx && y >= 0 && y < g.ny && z >= 0 && z < g.nz;
         const long long m = ok ? b * vol + (long long)z * plane + (long long)y * g.nx + x : 0;
         const bf16x8 v = *reinterpret_cast<const bf16x8 *>(in + m * CIP + part * 8);
@@ -121,13 +133,13 @@ __global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ 
         *reinterpret_cast<bf16x8 *>(halo + hv * VS + part * 16) = ok ? v : zero8;
     }
     __syncthreads();
-    // this lane's operand rows: voxel (i, j, k) = (r & 7, 2 t + (r >> 3), w) of the tile
+    // this lane's operand rows
     int hbase[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        const int r = lane & 15;
-        const int i = r & 7, j = 2 * t + (r >> 3), k = w;
-        hbase[t] = ((k + 1) * kHY + (j + 1)) * kHX + (i + 1);
+        int i, j, k;
+        TL::voxel(w, t, lane & 15, i, j, k);
+        hbase[t] = ((k + 1) * TL::H + (j + 1)) * TL::H + (i + 1);
     }
     f32x4 acc[MT][NT];
 #pragma unroll
@@ -142,7 +154,7 @@ __global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ 
         const int o = cc / CH;
         const int ci0 = (cc - o * CH) * 8;
         const int dz = o / 9 - 1, dy = (o / 3) % 3 - 1, dx = o % 3 - 1;
-        const int doff = (dz * kHY + dy) * kHX + dx;
+        const int doff = (dz * TL::H + dy) * TL::H + dx;
         bf16x8 a[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
@@ -168,9 +180,9 @@ __global__ void __launch_bounds__(512) k_conv_t(Geo g, const bf16 *__restrict__ 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 // output row 4 grp + r of operand tile t
-                const int v = 4 * grp + r;
-                const int i = v & 7, j = 2 * t + (v >> 3), k = w;
-                const int x = sx + d * (tx * kTX + i), y = sy + d * (ty * kTY + j), z = sz + d * (tz * kTZ + k);
+                int i, j, k;
+                TL::voxel(w, t, 4 * grp + r, i, j, k);
+                const int x = sx + d * (tx * TE + i), y = sy + d * (ty * TE + j), z = sz + d * (tz * TE + k);
                 if (x >= g.nx || y >= g.ny || z >= g.nz) continue;
                 const long long mo = b * vol + (long long)z * plane + (long long)y * g.nx + x;
                 float val = acc[t][nt][r];
@@ -191,11 +203,20 @@ template <int CIP, int COP, int MODE>
 void launch_conv(const Geo &g, const bf16 *in, const bf16 *W, const float *bias, bf16 *out_bf, float *out_f,
                  const bf16 *mask, hipStream_t s)
 {
-    const TileGeo tg = tile_geo(g);
-    const long long grid = (long long)g.B * g.dil * g.dil * g.dil * tg.ntx * tg.nty * tg.ntz;
-    const size_t lds = (size_t)kHalo * CIP * 2;
-    hipLaunchKernelGGL((k_conv_t<CIP, COP, MODE>), dim3((unsigned)grid), dim3(512), lds, s, g, in, W, bias, out_bf,
-                       out_f, mask);
+    // Padded voxels of either tiling.  The small tile loads 3.4 halo voxels per output
+    // instead of 1.95, so it is taken where it at least halves them: a layer with
+    // dilation 8 on 32^3 (4^3 sub-grids) computed eight times its voxels (8 x 32^3,
+    // 32 to 32 channels: 150 -> 45 us forward, 155 -> 55 us backward; at dilation 1
+    // the large tile takes 29 us).
+    const long long subs = (long long)g.B * g.dil * g.dil * g.dil;
+    const TileGeo t8 = tile_geo(g, 8), t4 = tile_geo(g, 4);
+    const long long n8 = subs * t8.ntx * t8.nty * t8.ntz, n4 = subs * t4.ntx * t4.nty * t4.ntz;
+    if (n8 * 512 >= 2 * n4 * 64)
+        hipLaunchKernelGGL((k_conv_t<CIP, COP, MODE, 4>), dim3((unsigned)n4), dim3(64 * Tile<4>::waves),
+                           (size_t)Tile<4>::halo * CIP * 2, s, g, in, W, bias, out_bf, out_f, mask);
+    else
+        hipLaunchKernelGGL((k_conv_t<CIP, COP, MODE, 8>), dim3((unsigned)n8), dim3(64 * Tile<8>::waves),
+                           (size_t)Tile<8>::halo * CIP * 2, s, g, in, W, bias, out_bf, out_f, mask);
 }
 
 // ---------------------------------------------------------------------------
