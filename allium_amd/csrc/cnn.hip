@@ -220,203 +220,191 @@ void launch_conv(const Geo &g, const bf16 *in, const bf16 *W, const float *bias,
 }
 
 // ---------------------------------------------------------------------------
-// weight gradient partials: part[plane][27][COP][CIT]
+// weight and bias gradient partials: part[workgroup][28][COP][CIP]; entry 27 is the
+// bias gradient in every column
 // ---------------------------------------------------------------------------
-// One workgroup per (batch, z) plane; K steps of 32 voxels along x, row by row.
-// Each step stages the step's gradient rows transposed (gT[co][x]) and the
-// nine (dz, dy) input rows with a dil-voxel halo each side (aT[r9][ci][x]) in
-// LDS.  The global reads are 16-byte channel chunks; those of the next step are
-// issued into registers before this step's MFMAs, so their latency hides
-// behind them.  A thread stages two neighbouring input voxels, so each channel
-// pair goes to LDS as one 4-byte store.  Row strides are padded: gT's keeps
-// 16-byte operand reads aligned and spreads its 16 rows over the banks, aT's is
-// an odd number of dwords.
-template <int CIP, int COP>
-__global__ void __launch_bounds__(256) k_wgrad(Geo g, const bf16 *__restrict__ gz, const bf16 *__restrict__ a,
-                                               float *__restrict__ part)
+// eight voxels of the lane's channel: two transposing reads of 4 voxels x 16 channels
+// per 16 lanes (lane 4 v + c of a group gives voxel v, channels 4 c .. 4 c + 3, and
+// receives channel 4 v + c of the four voxels); every lane of the wave takes part
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x8 tr_pair(const bf16 *lo, const bf16 *hi)
 {
-    constexpr int NTO = COP / 16, NTI = (CIP + 15) / 16, CIT = NTI * 16, NPAIR = NTO * NTI;
-    constexpr int XW = 32;                        // voxels per K step
-    constexpr int XSMAX = XW + 2 * kMaxDil;       // staged x range (dil-voxel halo each side)
-    constexpr int GS = XW + 8, AS = XSMAX + 2;    // LDS row strides (bf16)
-    constexpr int CHI = CIP / 8, CHO = COP / 8;   // 16-byte chunks per voxel
-    constexpr int NA = (9 * (XSMAX / 2) * CHI + 255) / 256, NG = (XW * CHO + 255) / 256;
-    static_assert(NPAIR == 1 || NPAIR == 2 || NPAIR == 4, "tile pairs divide the four waves");
-    // The waves take the NPAIR (16 co x 16 ci) tile pairs.  With 8 input
-    // channels, the waves left over share a pair and split its 27 taps (input
-    // layer: 126 -> 86 us on 8 x 32^3); with 32 they stay idle, which timed
-    // faster than splitting.
-    constexpr int WPP = CIP <= 8 ? 4 / NPAIR : 1;
-    __shared__ __attribute__((aligned(16))) bf16 gT[COP][GS];
-    __shared__ __attribute__((aligned(16))) bf16 aT[9][CIP][AS];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, grp = lane >> 4;
-    const int plane = blockIdx.x;
-    const int b = plane / g.nz, z = plane - b * g.nz;
-    const bool active = w < NPAIR * WPP;
-    const int pw = WPP == 1 ? w : w % NPAIR, tap0 = WPP == 1 ? 0 : w / NPAIR;   // taps o = tap0 mod WPP
-    const int cot = active ? pw / NTI : 0, cit = active ? pw % NTI : 0;
-    const int dl = g.dil, xr = XW + 2 * dl;
-    const int nxs = (g.nx + XW - 1) / XW, nsteps = g.ny * nxs;
-    const long long plane_base = ((long long)b * g.nz + z) * g.ny * g.nx;
-    const bf16x8 zero8 = {};
-    bf16x8 ra[NA][2], rg[NG];
-    const int xh = xr / 2;
-    // the step's global reads into registers; out-of-grid and padding chunks read
-    // voxel 0 and are zeroed by a select
-    auto load = [&](int st) {
-        const int y = st / nxs, x0 = (st - y * nxs) * XW;
-#pragma unroll
-        for (int k = 0; k < NG; ++k) {
-            const int i = threadIdx.x + 256 * k;
-            const int xi = i / CHO, c = i - xi * CHO;
-            const bool ok = i < XW * CHO && x0 + xi < g.nx;
-            const long long v = ok ? plane_base + (long long)y * g.nx + x0 + xi : 0;
+    using lds4 = __attribute__((address_space(3))) bf16x4;
+    const bf16x4 l = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4 *)lo);
+    const bf16x4 h = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4 *)hi);
+    return __builtin_shufflevector(l, h, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+constexpr int kWgradWaves = 8;
+
+// nshare workgroups per (batch, z) plane, which divide its dilation residues of
+// y, or its rows where there are fewer residues than shares.  A K step is 32
+// voxels of a row; the rows are taken in chains y, y + dil, y + 2 dil, ..., so
+// that a step finds two of the three input rows of each of its z planes in LDS (a
+// ring of four row sets) and stages one: a third of the reads.  Rows stay in
+// memory order (voxel, channel): the matrix operands need eight voxels of one
+// channel per lane, which ds_read_b64_tr_b16 takes from four voxels by sixteen
+// channels at any voxel offset, so the dx shifts cost nothing.  (With rows
+// transposed by the stores and eight 2-byte reads per shifted operand, the LDS
+// reads took 116 us of 8 x 32^3, 32 to 32 channels, at 256 workgroups of four
+// waves; now 45 us.) The next step's global reads are in flight in registers
+// during this step's MFMAs (two steps ahead timed the same); as a store only
+// touches the ring's fourth set, one barrier per step is enough.  Eight waves
+// share the operand tiles (16 input channels of a tap, or with 8 input channels
+// two taps), each for all output channels.
+template <int CIP, int COP>
+__global__ void __launch_bounds__(64 * kWgradWaves) k_wgrad(Geo g, int nshare, const bf16 *__restrict__ gz,
+                                               const bf16 *__restrict__ a, float *__restrict__ part)
+{
+    constexpr int NW = kWgradWaves, NTH = 64 * NW, NTO = COP / 16, NTI = (CIP + 15) / 16;
+    constexpr int TPT = CIP < 16 ? 16 / CIP : 1;          // taps per operand tile
+    constexpr int WT = NW / NTI;                          // waves over the taps of an input channel tile
+    constexpr int NTT = (27 + TPT - 1) / TPT, NB = (NTT + WT - 1) / WT;   // tap tiles, and per wave
+    constexpr int XW = 32, XS = XW + 2 * kMaxDil;         // voxels per K step, staged per row
+    constexpr int CHI = CIP / 8, CHO = COP / 8;           // 16-byte chunks per voxel
+    constexpr int AV = CIP, GV = COP;   // LDS voxel strides (bf16)
+    constexpr int NA = (3 * XS * CHI + NTH - 1) / NTH;
+    static_assert(NTT * TPT > 27 || NB * WT * TPT > 27, "a tile is left for the bias gradient");
+    static_assert(XW * CHO <= NTH && NW % NTI == 0 && (TPT == 1 || NTI == 1), "one chunk of gz per thread; tiles divide the waves");
+    __shared__ __attribute__((aligned(16))) bf16 gR[2][XW * GV];
+    __shared__ __attribute__((aligned(16))) bf16 aR[4][3][XS * AV];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int share = blockIdx.x % nshare, pl = blockIdx.x / nshare, z = pl % g.nz, b = pl / g.nz;
+    const int dl = g.dil, xr = XW + 2 * dl, nxs = (g.nx + XW - 1) / XW;
+    const bool by_res = min(dl, g.ny) >= nshare;
+    const int ya = by_res ? 0 : (int)((long long)g.ny * share / nshare);
+    const int yb = by_res ? g.ny : (int)((long long)g.ny * (share + 1) / nshare);
+    const int r0 = by_res ? share : 0, dr = by_res ? nshare : 1, r1 = min(dl, yb - ya);
+    const bf16x8 zero8 = {}, one8 = zero8 + (bf16)1.f;
+    struct Regs { bf16x8 a[NA], g; } q;
+    // position in the share's steps: x chunk, y residue, row
+    struct Pos { int xs, r, y; };
+    // reads of a step into registers: gradient row y, input rows y + dil of the three
+    // planes; out-of-grid chunks read voxel 0 and are zeroed by a select
+    auto load = [&](const Pos &p) {
+        const int x0 = p.xs * XW, y = p.y;
+        {
+            const int xi = threadIdx.x / CHO, c = threadIdx.x % CHO;
+            const bool ok = xi < XW && x0 + xi < g.nx && y >= ya;
+            const long long v = ok ? (((long long)b * g.nz + z) * g.ny + y) * g.nx + x0 + xi : 0;
             const bf16x8 r = *reinterpret_cast<const bf16x8 *>(gz + v * COP + 8 * c);
-            rg[k] = ok ? r : zero8;
+            q.g = ok ? r : zero8;
         }
+        const int yy = y + dl;
 #pragma unroll
         for (int k = 0; k < NA; ++k) {
-            const int i = threadIdx.x + 256 * k;
+            const int i = threadIdx.x + NTH * k;
             const int c = i % CHI, rest = i / CHI;
-            const int xp = rest % xh, r9 = rest / xh;
-            const int yy = y + (r9 % 3 - 1) * dl, zz = z + (r9 / 3 - 1) * dl;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int xx = x0 - dl + 2 * xp + h;
-                const bool ok = r9 < 9 && xx >= 0 && xx < g.nx && yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz;
-                const long long v = ok ? (((long long)b * g.nz + zz) * g.ny + yy) * g.nx + xx : 0;
-                const bf16x8 r = *reinterpret_cast<const bf16x8 *>(a + v * CIP + 8 * c);
-                ra[k][h] = ok ? r : zero8;
-            }
+            const int xp = rest % XS, r3 = rest / XS;
+            const int xx = x0 - dl + xp, zz = z + (r3 - 1) * dl;
+            const bool ok = r3 < 3 && xp < xr && xx >= 0 && xx < g.nx && yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz;
+            const long long v = ok ? (((long long)b * g.nz + zz) * g.ny + yy) * g.nx + xx : 0;
+            const bf16x8 r = *reinterpret_cast<const bf16x8 *>(a + v * CIP + 8 * c);
+            q.a[k] = ok ? r : zero8;
         }
     };
-    f32x4 acc[27];
+    // this lane's part of the transposing reads: voxel and channel chunk of its 16-lane
+    // group's 4 x 16 block (the group holds voxels 8 grp .. 8 grp + 7 of the step)
+    const int rv = 8 * (lane >> 4) + ((lane & 15) >> 2), rc = lane & 3;
+    const int cit = w % NTI, tap0 = w / NTI;
+    int aoff[NB], adz[NB], ady[NB];
 #pragma unroll
-    for (int o = 0; o < 27; ++o) acc[o] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (nsteps > 0) load(0);
-    for (int st = 0; st < nsteps; ++st) {
-        __syncthreads();   // the previous step's operand reads are done
+    for (int i = 0; i < NB; ++i) {
+        int o = (tap0 + i * WT) * TPT + (TPT > 1 ? 4 * rc / CIP : 0);
+        o = o < 27 ? o : 26;
+        adz[i] = o / 9;
+        ady[i] = (o / 3) % 3 - 1;
+        aoff[i] = (rv + dl * (o % 3)) * AV + (TPT > 1 ? (4 * rc) % CIP : cit * 16 + 4 * rc);
+    }
+    f32x4 acc[NTO][NB];
 #pragma unroll
-        for (int k = 0; k < NG; ++k) {
-            const int i = threadIdx.x + 256 * k;
-            if (i < XW * CHO) {
-                const int xi = i / CHO, c = i - xi * CHO;
+    for (int m = 0; m < NTO; ++m)
 #pragma unroll
-                for (int t = 0; t < 8; ++t) gT[8 * c + t][xi] = rg[k][t];
-            }
+        for (int i = 0; i < NB; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // a chain (x chunk, y residue r) opens with two steps that only stage rows
+    // ya + r - dil and ya + r
+    Pos cp = {r1 > r0 ? 0 : nxs, r0, ya + r0 - 2 * dl};
+    auto advance = [&](Pos &p) {
+        p.y += dl;
+        if (p.y >= yb) {
+            p.r += dr;
+            if (p.r >= r1) { p.r = r0; ++p.xs; }
+            p.y = ya + p.r - 2 * dl;
         }
+    };
+    if (cp.xs < nxs) load(cp);
+    for (int e = 0; cp.xs < nxs; ++e) {
+        if (threadIdx.x < XW * CHO)
+            *reinterpret_cast<bf16x8 *>(&gR[e & 1][(threadIdx.x / CHO) * GV + 8 * (threadIdx.x % CHO)]) = q.g;
 #pragma unroll
         for (int k = 0; k < NA; ++k) {
-            const int i = threadIdx.x + 256 * k;
+            const int i = threadIdx.x + NTH * k;
             const int c = i % CHI, rest = i / CHI;
-            const int xp = rest % xh, r9 = rest / xh;
-            if (r9 < 9) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    *reinterpret_cast<bf16x2 *>(&aT[r9][8 * c + t][2 * xp]) = bf16x2{ra[k][0][t], ra[k][1][t]};
-            }
+            const int xp = rest % XS, r3 = rest / XS;
+            if (r3 < 3) *reinterpret_cast<bf16x8 *>(&aR[e & 3][r3][xp * AV + 8 * c]) = q.a[k];
         }
         __syncthreads();
-        if (st + 1 < nsteps) load(st + 1);
-        if (active) {
-            const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&gT[cot * 16 + (lane & 15)][8 * grp]);
-            const int ci = cit * 16 + (lane & 15);
+        const bool compute = cp.y >= ya;
+        advance(cp);
+        if (cp.xs < nxs) load(cp);
+        if (!compute) continue;
+        bf16x8 av[NTO];
 #pragma unroll
-            for (int o = 0; o < 27; ++o) {
-                if (WPP > 1 && o % WPP != tap0) continue;
-                const int dz = o / 9 - 1, dy = (o / 3) % 3 - 1, dx = o % 3 - 1;
-                const int r9 = (dz + 1) * 3 + (dy + 1);
-                bf16x8 bv;
+        for (int m = 0; m < NTO; ++m) {
+            const bf16 *p = &gR[e & 1][rv * GV + m * 16 + 4 * rc];
+            av[m] = tr_pair(p, p + 4 * GV);
+        }
 #pragma unroll
-                for (int t = 0; t < 8; ++t) bv[t] = ci < CIP ? aT[r9][ci][dl * (1 + dx) + 8 * grp + t] : (bf16)0.f;
-                acc[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[o], 0, 0, 0);
-            }
+        for (int i = 0; i < NB; ++i) {
+            const bf16 *p = &aR[(e - 1 + ady[i]) & 3][adz[i]][aoff[i]];
+            bf16x8 bv = tr_pair(p, p + 4 * AV);
+            // the tap after the last multiplies by ones: the bias gradient
+            if ((tap0 + i * WT) * TPT + (TPT > 1 ? (lane & 15) / CIP : 0) == 27) bv = one8;
+#pragma unroll
+            for (int m = 0; m < NTO; ++m)
+                acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv, acc[m][i], 0, 0, 0);
         }
     }
-    if (!active) return;
 #pragma unroll
-    for (int o = 0; o < 27; ++o) {
-        if (WPP > 1 && o % WPP != tap0) continue;
+    for (int i = 0; i < NB; ++i) {
+        const int n = lane & 15, o = (tap0 + i * WT) * TPT + (TPT > 1 ? n / CIP : 0);
+        const int ci = TPT > 1 ? n % CIP : cit * 16 + n;
+        if (o > 27) continue;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int co = cot * 16 + 4 * grp + r, ci = cit * 16 + (lane & 15);
-            part[(((long long)plane * 27 + o) * COP + co) * CIT + ci] = acc[o][r];
-        }
+        for (int m = 0; m < NTO; ++m)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                part[(((long long)blockIdx.x * 28 + o) * COP + m * 16 + 4 * (lane >> 4) + q) * CIP + ci] = acc[m][i][q];
     }
 }
 
-// grad[o][co][ci] (packed, real sizes) = sum over planes of the partials.  A
-// block sums 64 outputs: each of its four waves adds every fourth plane (loads
-// unrolled eight deep) and the four sums are added in wave order, so the result
-// does not depend on timing.
-__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, int nplane, int COP, int CIT,
+// grad[o][co][ci], then the bias gradient [co] (packed, real sizes) = sums of the
+// partials.  A block sums 64 outputs: each of its four waves adds every fourth
+// partial in four chains (sixteen loads in flight) and the sums are added in a fixed
+// order, so the result does not depend on timing.
+__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, int nparts, int COP, int CIP,
                                                       int CO, int CI, float *__restrict__ grad)
 {
     __shared__ float red[4][64];
-    const int n = 27 * CO * CI;
+    const int nw = 27 * CO * CI, n = nw + CO;
     const int jl = threadIdx.x & 63, sl = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + jl;
-    float s = 0.f;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
     if (i < n) {
-        const int o = i / (CO * CI), rem = i - o * CO * CI, co = rem / CI, ci = rem - co * CI;
-        const long long stride = 27LL * COP * CIT;
-        const float *p0 = part + ((long long)o * COP + co) * CIT + ci;
-#pragma unroll 8
-        for (int p = sl; p < nplane; p += 4) s += p0[p * stride];
+        const int o = i < nw ? i / (CO * CI) : 27, rem = i - o * CO * CI;
+        const int co = i < nw ? rem / CI : rem, ci = i < nw ? rem - co * CI : 0;
+        const long long stride = 28LL * COP * CIP;
+        const float *p0 = part + ((long long)o * COP + co) * CIP + ci;
+        int p = sl;
+#pragma unroll 4
+        for (; p + 12 < nparts; p += 16)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s[k] += p0[(p + 4 * k) * stride];
+        for (; p < nparts; p += 4) s[0] += p0[p * stride];
     }
-    red[sl][jl] = s;
+    red[sl][jl] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
     if (sl == 0 && i < n) grad[i] = ((red[0][jl] + red[1][jl]) + red[2][jl]) + red[3][jl];
-}
-
-// bias gradient partials: bpart[block][COP] = sum over the block's voxels.  A
-// thread reads one 16-byte chunk (8 channels) of a voxel per step; the block's
-// per-thread sums are added in a fixed order.
-template <int COP>
-__global__ void __launch_bounds__(256) k_bias_grad(long long T, const bf16 *__restrict__ gz, float *__restrict__ bpart)
-{
-    constexpr int CHO = COP / 8, VPB = 256 / CHO;
-    __shared__ float red[256][9];
-    const int c = threadIdx.x % CHO, vi = threadIdx.x / CHO;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (long long v = (long long)blockIdx.x * VPB + vi; v < T; v += (long long)gridDim.x * VPB) {
-        const bf16x8 r = *reinterpret_cast<const bf16x8 *>(gz + v * COP + 8 * c);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) s[t] += (float)r[t];
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) red[threadIdx.x][t] = s[t];
-    __syncthreads();
-    if (threadIdx.x < COP) {
-        const int cc = threadIdx.x >> 3, t = threadIdx.x & 7;
-        float a = 0.f;
-        for (int k = 0; k < VPB; ++k) a += red[k * CHO + cc][t];
-        bpart[(long long)blockIdx.x * COP + threadIdx.x] = a;
-    }
-}
-
-// grad[co] = sum over the partials of k_bias_grad: eight slices of 32 threads
-// (one per channel) add every eighth partial, then the slices in order
-__global__ void __launch_bounds__(256) k_bias_reduce(const float *__restrict__ bpart, int nblk, int COP, int CO,
-                                                     float *__restrict__ grad)
-{
-    static_assert(HID <= 32, "one thread per channel in a 32-thread slice");
-    __shared__ float red[8][32];
-    const int co = threadIdx.x & 31, sl = threadIdx.x >> 5;
-    float s = 0.f;
-    if (co < CO) {
-#pragma unroll 8
-        for (int b = sl; b < nblk; b += 8) s += bpart[(long long)b * COP + co];
-    }
-    red[sl][co] = s;
-    __syncthreads();
-    if (sl == 0 && co < CO) {
-        float a = 0.f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) a += red[k][co];
-        grad[co] = a;
-    }
 }
 
 // x [T][3] float -> [T][8] bf16
@@ -605,9 +593,9 @@ struct allium_cnn {
     float *bias[NL] = {};
     bool packed = false;
     long long cap = 0;
-    int cap_planes = 0;
+    int cap_parts = 0;   // weight-gradient partials
     bf16 *xin = nullptr, *act[NL - 1] = {}, *ga = nullptr, *gb = nullptr;
-    float *out = nullptr, *part = nullptr, *bpart = nullptr, *xf = nullptr;
+    float *out = nullptr, *part = nullptr, *xf = nullptr;
     double *lpart = nullptr, *ravg = nullptr, *rpart = nullptr, *scale = nullptr;
     long step = 0;
     int dil[NL] = {1, 1, 1, 1, 1};
@@ -629,13 +617,22 @@ struct allium_cnn {
 
 namespace {
 
-constexpr int kBiasBlocks = 256;
+constexpr int kWgradGroups = 256;
 constexpr int kLossBlocks = 512;
+
+// workgroups per plane of the weight gradients: one per CU in all, up to four per
+// plane (on 8 x 32^3, 256 planes, two per CU took 39 instead of 45 us a layer, but
+// their partials' sum 18 instead of 10 us; sixteen waves instead of eight took 49 us)
+int wgrad_shares(const Geo &g)
+{
+    const long long want = kWgradGroups / ((long long)g.B * g.nz);
+    return (int)(want < 1 ? 1 : want > 4 ? 4 : want);
+}
 
 int ensure(allium_cnn *h, const Geo &g)
 {
-    const int planes = g.B * g.nz;
-    if (g.T <= h->cap && planes <= h->cap_planes) return 0;
+    int parts = g.B * g.nz * wgrad_shares(g);
+    if (g.T <= h->cap && parts <= h->cap_parts) return 0;
     // grow: free the old work buffers by re-creating the list
     std::vector<void *> keep;
     for (void *p : h->owned) {
@@ -646,7 +643,9 @@ int ensure(allium_cnn *h, const Geo &g)
         else keep.push_back(p);
     }
     h->owned = keep;
-    const long long T = g.T;
+    // neither size shrinks: calls that alternate between shapes settle
+    const long long T = g.T > h->cap ? g.T : h->cap;
+    if (parts < h->cap_parts) parts = h->cap_parts;
     CNN_TRY(h->alloc(&h->xin, (size_t)T * 8));
     for (int l = 0; l < NL - 1; ++l) CNN_TRY(h->alloc(&h->act[l], (size_t)T * HID));
     CNN_TRY(h->alloc(&h->ga, (size_t)T * HID));
@@ -654,9 +653,9 @@ int ensure(allium_cnn *h, const Geo &g)
     CNN_TRY(h->alloc(&h->out, (size_t)T));
     CNN_TRY(h->alloc(&h->xf, (size_t)T * 3));
     CNN_TRY(h->alloc(&h->ravg, (size_t)T));
-    CNN_TRY(h->alloc(&h->part, (size_t)planes * 27 * 32 * 32));
+    CNN_TRY(h->alloc(&h->part, (size_t)parts * 28 * 32 * 32));
     h->cap = T;
-    h->cap_planes = planes;
+    h->cap_parts = parts;
     return 0;
 }
 
@@ -716,29 +715,23 @@ int gradient(allium_cnn *h, const Geo &g, const float *d_x, const float *d_t, do
     rc = forward_packed(h, g, s);
     if (rc) return rc;
     hipLaunchKernelGGL(k_loss, dim3(kLossBlocks), dim3(256), 0, s, g.T, h->out, d_t, h->ga, h->lpart);
-    const int planes = g.B * g.nz;
+    const int planes = g.B * g.nz, nshare = wgrad_shares(g);
     // layer 5: gz = ga [T][16]
     const bf16 *gz = h->ga;
     bf16 *gnext = h->gb;
     for (int l = NL - 1; l >= 0; --l) {
         const bf16 *ain = l == 0 ? h->xin : h->act[l - 1];
         float *gW = h->grad + layer_offset(l);
-        float *gB = gW + 27L * CO_[l] * CI_[l];
-        const int CIT = ((CIP_[l] + 15) / 16) * 16;
         const Geo gl = layer_geo(h, g, l);
         if (l == NL - 1) {
-            hipLaunchKernelGGL((k_wgrad<32, 16>), dim3(planes), dim3(256), 0, s, gl, gz, ain, h->part);
-            hipLaunchKernelGGL(k_bias_grad<16>, dim3(kBiasBlocks), dim3(256), 0, s, g.T, gz, h->bpart);
+            hipLaunchKernelGGL((k_wgrad<32, 16>), dim3(planes * nshare), dim3(64 * kWgradWaves), 0, s, gl, nshare, gz, ain, h->part);
         } else if (l == 0) {
-            hipLaunchKernelGGL((k_wgrad<8, 32>), dim3(planes), dim3(256), 0, s, gl, gz, ain, h->part);
-            hipLaunchKernelGGL(k_bias_grad<32>, dim3(kBiasBlocks), dim3(256), 0, s, g.T, gz, h->bpart);
+            hipLaunchKernelGGL((k_wgrad<8, 32>), dim3(planes * nshare), dim3(64 * kWgradWaves), 0, s, gl, nshare, gz, ain, h->part);
         } else {
-            hipLaunchKernelGGL((k_wgrad<32, 32>), dim3(planes), dim3(256), 0, s, gl, gz, ain, h->part);
-            hipLaunchKernelGGL(k_bias_grad<32>, dim3(kBiasBlocks), dim3(256), 0, s, g.T, gz, h->bpart);
+            hipLaunchKernelGGL((k_wgrad<32, 32>), dim3(planes * nshare), dim3(64 * kWgradWaves), 0, s, gl, nshare, gz, ain, h->part);
         }
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((27L * CO_[l] * CI_[l] + 63) / 64)), dim3(256), 0, s,
-                           h->part, planes, COP_[l], CIT, CO_[l], CI_[l], gW);
-        hipLaunchKernelGGL(k_bias_reduce, dim3(1), dim3(256), 0, s, h->bpart, kBiasBlocks, COP_[l], CO_[l], gB);
+        hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((27L * CO_[l] * CI_[l] + CO_[l] + 63) / 64)), dim3(256), 0, s,
+                           h->part, planes * nshare, COP_[l], CIP_[l], CO_[l], CI_[l], gW);
         if (l > 0) {
             // gradient of the previous pre-activation: conv with flipped weights, ReLU mask of its output
             if (l == NL - 1)
@@ -837,7 +830,6 @@ int allium_cnn_create(unsigned long long seed, allium_cnn_t *out)
         if ((e = h->alloc(&h->Wb[l], 27L * COP_[l] * CIP_[l])) != hipSuccess) return bad(e);
         if ((e = h->alloc(&h->bias[l], COP_[l])) != hipSuccess) return bad(e);
     }
-    if ((e = h->alloc(&h->bpart, (size_t)kBiasBlocks * 32)) != hipSuccess) return bad(e);
     if ((e = h->alloc(&h->lpart, kLossBlocks)) != hipSuccess) return bad(e);
     if ((e = h->alloc(&h->rpart, 256)) != hipSuccess) return bad(e);
     if ((e = h->alloc(&h->scale, 1)) != hipSuccess) return bad(e);
