@@ -204,14 +204,15 @@ void launch_conv(const Geo &g, const bf16 *in, const bf16 *W, const float *bias,
                  const bf16 *mask, hipStream_t s)
 {
     // Padded voxels of either tiling.  The small tile loads 3.4 halo voxels per output
-    // instead of 1.95, so it is taken where it at least halves them: a layer with
+    // instead of 1.95, so it is taken where it more than halves them
+    // (at exactly half, a forward pass on 49 x 15 x 34 took 99 instead of 94 us): a layer with
     // dilation 8 on 32^3 (4^3 sub-grids) computed eight times its voxels (8 x 32^3,
     // 32 to 32 channels: 150 -> 45 us forward, 155 -> 55 us backward; at dilation 1
     // the large tile takes 29 us).
     const long long subs = (long long)g.B * g.dil * g.dil * g.dil;
     const TileGeo t8 = tile_geo(g, 8), t4 = tile_geo(g, 4);
     const long long n8 = subs * t8.ntx * t8.nty * t8.ntz, n4 = subs * t4.ntx * t4.nty * t4.ntz;
-    if (n8 * 512 >= 2 * n4 * 64)
+    if (n8 * 512 > 2 * n4 * 64)
         hipLaunchKernelGGL((k_conv_t<CIP, COP, MODE, 4>), dim3((unsigned)n4), dim3(64 * Tile<4>::waves),
                            (size_t)Tile<4>::halo * CIP * 2, s, g, in, W, bias, out_bf, out_f, mask);
     else
