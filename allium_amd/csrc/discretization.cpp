@@ -331,13 +331,16 @@ bool build_mesh(int dim, const int *nel, const double *vertices, const double *e
     }
     for (double x : m.vert)
         if (!std::isfinite(x)) { err = "non-finite vertex coordinate"; return false; }
-    // uniform axis-aligned box grid?
+    // uniform axis-aligned box grid?  Its kernels take the low side of every axis to
+    // be the one with the smaller coordinate, so a grid whose coordinates fall along
+    // an axis (turned by 180 degrees about another) is general geometry.
     m.uniform = true;
     for (int d = 0; d < dim; d++) {
         const double x0 = m.vert[d];
         const long last = (long)(m.nv[0] - 1) * (d == 0) + (long)m.nv[0] * (m.nv[1] - 1) * (d == 1) +
                           (long)m.nv[0] * m.nv[1] * (m.nv[2] - 1) * (d == 2);
         m.h[d] = (m.vert[last * dim + d] - x0) / m.nel[d];
+        if (!(m.h[d] > 0)) m.uniform = false;
     }
     for (long v = 0; v < nvt && m.uniform; v++) {
         const long c[3] = {v % m.nv[0], (v / m.nv[0]) % m.nv[1], v / ((long)m.nv[0] * m.nv[1])};

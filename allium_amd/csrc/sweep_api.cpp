@@ -233,7 +233,7 @@ int upload_all(allium_sweep *h)
         HIP_TRY(upload(ds.owned, &ds.d_cls_ptr, cls.data(), cls.size()));
         ds.angle_independent = h->plan.angle_independent;
         ds.lumped = ed.lump != 0;
-        for (int d = 0; d < 2; d++) ds.h2[d] = m.uniform ? std::fabs(m.h[d]) : 0.0;
+        for (int d = 0; d < 2; d++) ds.h2[d] = m.uniform ? m.h[d] : 0.0;
     }
     ds.level_ptr = h->plan.level_ptr;
     ds.nlevels = h->plan.nlevels;
