@@ -594,7 +594,7 @@ struct allium_cnn {
     float *bias[NL] = {};
     bool packed = false;
     long long cap = 0;
-    int cap_parts = 0;   // weight-gradient partials
+    long long cap_parts = 0;   // weight-gradient partials
     bf16 *xin = nullptr, *act[NL - 1] = {}, *ga = nullptr, *gb = nullptr;
     float *out = nullptr, *part = nullptr, *xf = nullptr;
     double *lpart = nullptr, *ravg = nullptr, *rpart = nullptr, *scale = nullptr;
@@ -630,33 +630,54 @@ int wgrad_shares(const Geo &g)
     return (int)(want < 1 ? 1 : want > 4 ? 4 : want);
 }
 
-int ensure(allium_cnn *h, const Geo &g)
+// the work buffers of T voxels and so many partials; after a failure the handle holds none
+hipError_t alloc_work(allium_cnn *h, long long T, long long parts)
 {
-    int parts = g.B * g.nz * wgrad_shares(g);
-    if (g.T <= h->cap && parts <= h->cap_parts) return 0;
-    // grow: free the old work buffers by re-creating the list
-    std::vector<void *> keep;
-    for (void *p : h->owned) {
-        bool work = p == h->xin || p == h->ga || p == h->gb || p == h->out || p == h->part || p == h->xf ||
-                    p == h->ravg;
-        for (int l = 0; l < NL - 1; ++l) work = work || p == h->act[l];
-        if (work) hipFree(p);
-        else keep.push_back(p);
+    auto free_work = [&] {
+        std::vector<void *> keep;
+        for (void *p : h->owned) {
+            bool work = p == h->xin || p == h->ga || p == h->gb || p == h->out || p == h->part || p == h->xf ||
+                        p == h->ravg;
+            for (int l = 0; l < NL - 1; ++l) work = work || p == h->act[l];
+            if (work) hipFree(p);
+            else keep.push_back(p);
+        }
+        h->owned = keep;
+        h->xin = h->ga = h->gb = nullptr;
+        h->out = h->part = h->xf = nullptr;
+        h->ravg = nullptr;
+        for (bf16 *&a : h->act) a = nullptr;
+        h->cap = h->cap_parts = 0;
+    };
+    free_work();
+    hipError_t e = h->alloc(&h->xin, (size_t)T * 8);
+    for (int l = 0; l < NL - 1 && e == hipSuccess; ++l) e = h->alloc(&h->act[l], (size_t)T * HID);
+    if (e == hipSuccess) e = h->alloc(&h->ga, (size_t)T * HID);
+    if (e == hipSuccess) e = h->alloc(&h->gb, (size_t)T * HID);
+    if (e == hipSuccess) e = h->alloc(&h->out, (size_t)T);
+    if (e == hipSuccess) e = h->alloc(&h->xf, (size_t)T * 3);
+    if (e == hipSuccess) e = h->alloc(&h->ravg, (size_t)T);
+    if (e == hipSuccess) e = h->alloc(&h->part, (size_t)parts * 28 * 32 * 32);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // or the next launch's check reports it
+        free_work();
+        return e;
     }
-    h->owned = keep;
-    // neither size shrinks: calls that alternate between shapes settle
-    const long long T = g.T > h->cap ? g.T : h->cap;
-    if (parts < h->cap_parts) parts = h->cap_parts;
-    CNN_TRY(h->alloc(&h->xin, (size_t)T * 8));
-    for (int l = 0; l < NL - 1; ++l) CNN_TRY(h->alloc(&h->act[l], (size_t)T * HID));
-    CNN_TRY(h->alloc(&h->ga, (size_t)T * HID));
-    CNN_TRY(h->alloc(&h->gb, (size_t)T * HID));
-    CNN_TRY(h->alloc(&h->out, (size_t)T));
-    CNN_TRY(h->alloc(&h->xf, (size_t)T * 3));
-    CNN_TRY(h->alloc(&h->ravg, (size_t)T));
-    CNN_TRY(h->alloc(&h->part, (size_t)parts * 28 * 32 * 32));
     h->cap = T;
     h->cap_parts = parts;
+    return hipSuccess;
+}
+
+int ensure(allium_cnn *h, const Geo &g)
+{
+    const long long parts = (long long)g.B * g.nz * wgrad_shares(g);
+    if (g.T <= h->cap && parts <= h->cap_parts) return 0;
+    // neither size shrinks, so calls that alternate between shapes settle, unless the
+    // memory only holds what this call needs
+    const long long T1 = g.T > h->cap ? g.T : h->cap, parts1 = parts > h->cap_parts ? parts : h->cap_parts;
+    hipError_t e = alloc_work(h, T1, parts1);
+    if (e != hipSuccess && (T1 > g.T || parts1 > parts)) e = alloc_work(h, g.T, parts);
+    if (e != hipSuccess) return cfail(-4, std::string("network work buffers: ") + hipGetErrorString(e));
     return 0;
 }
 
