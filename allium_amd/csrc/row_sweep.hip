@@ -12,14 +12,21 @@
 // Cell solve.  With t_d = |Omega_d| / h_d, the mass m and the upwind convection C
 // of the unit interval, B = m^-1 C, the cell system times the inverse unit mass is
 //   vol (t_x B (x) I + t_y I (x) B + sigma).
-// B = V L V^-1 with L real: one eigenvalue l0 (p = 2) and a pair a +- i b as
-// [[a, b], [-b, a]].  At p = 2 they are the roots of x^3 - 9 x^2 + 36 x - 60, the
-// condition of V is 7.  In that basis of both axes the system falls into scalars,
-// 2 x 2 rotations and, for pair and pair, two 2 x 2 rotations in the +- eigenspaces
-// of the product of the two axes' J = [[0, 1], [-1, 0]].  The traces are passed on in
-// the basis of their own axis, so a step's chain from trace to trace is 2 Q^2
-// multiply-adds, the rotations, and 2 Q^2 more; the transform of the source, the
+// B = V L V^-1 with L real: a pair of eigenvalues a +- i b as [[a, b], [-b, a]] and, at
+// p = 2, a real one l0 (the roots of x^3 - 9 x^2 + 36 x - 60) that the pair couples
+// into: L = [[l0, 1, t], [0, a, b], [0, -b, a]], the real Schur form.  In that basis
+// of both axes the system is solved from the pair (x) pair unknowns (two 2 x 2
+// rotations in the +- eigenspaces of the product of the two axes' J = [[0, 1], [-1, 0]])
+// over pair (x) real (a rotation each) to real (x) real.  V is orthogonal under m but for
+// the ratio of the pair's two scales (1.9 at p = 1, 1.7 at p = 2).  The traces are passed
+// on in the basis of their own axis, so a step's chain from trace to trace is 2 Q^2
+// multiply-adds, the solve, and a few additions; the transform of the source, the
 // reciprocals and the transform to nodal values hang off it.
+//
+// Error (2-norm against extended precision, log-normal sigma): that of the LU within a
+// third at p = 2 (2.3e-15 on 150 x 97, LU 2.9e-15); a basis of eigenvectors
+// (condition 7 per axis) needs 12 instructions fewer and was at 1.5e-14.  At p = 1 3.7e-15
+// (LU 2.6e-15, box sweeps 2.0e-14): the pair's unknowns are three times their trace.
 //
 // Bound by issue: about 330 (p = 2) and 150 (p = 1) instructions a step in each of a
 // few waves per CU, one per about 8 cycles.  A 9 x 9 LU in one lane with the traces
@@ -35,31 +42,62 @@ namespace allium {
 
 namespace {
 
+// A trace that crosses an element is multiplied by r(z) = V_P (L + z)^-1 W0 (last row
+// of V, first column of W), and a rounding of their constants errs with one sign in
+// every element.  So some of them are neighbours (one unit in the last place) of the
+// nearest doubles: V11 at p = 1, which leaves 4e-17 instead of 2.7e-16 (z = 0), and t,
+// W00 and W20 at p = 2, 5e-18 instead of 1.3e-16.
 template <int P>
-struct Eig;
+struct Basis;
 template <>
-struct Eig<1> {
+struct Basis<1> {
     static constexpr int R = 0;   // real eigenvalues
-    static constexpr double l0 = 0.0, a = 2.0, b = 1.41421356237309504880;
-    static constexpr double V[2][2] = {{1.0, 0.0}, {-1.0, 1.41421356237309504880}};
-    static constexpr double W[2][2] = {{4.0, -2.0}, {1.41421356237309504880, 1.41421356237309504880}};   // V^-1 m^-1
+    static constexpr double l0 = 0.0, a = 2.0, b = 1.4142135623730950488, t = 0.0;
+    static constexpr double V[2][2] = {{1.0, 0.0}, {-1.0, 1.4142135623730949234}};
+    static constexpr double W[2][2] = {{4.0, -2.0}, {1.4142135623730950488, 1.4142135623730950488}};   // V^-1 m^-1
 };
 template <>
-struct Eig<2> {
+struct Basis<2> {
     static constexpr int R = 1;
-    // A trace that crosses an element is multiplied by
-    // r(z) = W00 / (l0 + z) + ((a + z) W10 - b W20) / ((a + z)^2 + b^2), with terms of 5 and
-    // -4 for a value of 1: its constants rounded to nearest leave 4.9e-16 in every
-    // element, always with one sign.  These are neighbours of the nearest doubles
-    // (within 3 units in the last place) with r exact to 4e-17, 5e-18 at z = 0.
-    static constexpr double l0 = 3.6378342527444953, a = 2.6810828736277528, b = 3.0504301992474105;
-    static constexpr double V[3][3] = {{0.257433446063711987, -0.06871672303185599, 0.388146850560913172},
-                                       {0.097974882877588054, 0.011012558561205972, -0.37446069925093946},
-                                       {1.0, 1.0, 0.0}};
-    static constexpr double W[3][3] = {{18.297498174845845, 1.792695240633402691, 4.710388009495045932},
-                                       {-15.297498174845845, -3.29269524063340269, 4.289611990504954067},
-                                       {8.34328048949488, -5.63643099835961522, 5.364352843454024324}};
+    static constexpr double l0 = 3.6378342527444958, a = 2.6810828736277523, b = 3.0504301992474105;
+    static constexpr double t = 0.24964484560420097115;
+    static constexpr double V[3][3] = {{2.2420123818119873, 1.0734624624372482, 1.2377295589054893},
+                                       {0.85327257928935929, -1.0240820485688007, -0.068423170697841346},
+                                       {8.7090951703964432, 1.0, 0.0}};
+    static constexpr double W[3][3] = {{0.2016957935665358026, 0.076762060461610951, 0.78348713677483162},
+                                       {1.2434121383604055, -2.1685280900358954, 2.1765359610465764},
+                                       {5.8276375688838841782, 0.52978617878836110, -0.88308266220483422}};
 };
+
+// largest deviation of W m V from I and of W C V from L
+template <int P>
+constexpr double basis_error()
+{
+    using E = Basis<P>;
+    constexpr int Q = P + 1, R = E::R;
+    constexpr double d1[2][2] = {{0.5, 0.5}, {-0.5, 0.5}};   // C: -(integral of phi_i' phi_j), + 1 at the last node
+    constexpr double d2[3][3] = {{0.5, 2.0 / 3.0, -1.0 / 6.0}, {-2.0 / 3.0, 0.0, 2.0 / 3.0}, {1.0 / 6.0, -2.0 / 3.0, 0.5}};
+    double worst = 0.0;
+    for (int i = 0; i < Q; ++i)
+        for (int j = 0; j < Q; ++j) {
+            double id = i == j ? -1.0 : 0.0, l = 0.0;
+            if (i >= R && j >= R) l = i == j ? E::a : (i < j ? E::b : -E::b);
+            else if (i < R) l = j == 0 ? E::l0 : (j == 1 ? 1.0 : E::t);
+            l = -l;
+            for (int k = 0; k < Q; ++k)
+                for (int n = 0; n < Q; ++n) {
+                    double c = 0.0;
+                    if constexpr (P == 1) c = d1[k][n];
+                    else c = d2[k][n];
+                    id += E::W[i][k] * unit_mass_1d<P>(k, n) * E::V[n][j];
+                    l += E::W[i][k] * c * E::V[n][j];
+                }
+            worst = id > worst ? id : (-id > worst ? -id : worst);
+            worst = l > worst ? l : (-l > worst ? -l : worst);
+        }
+    return worst;
+}
+static_assert(basis_error<1>() < 4e-15 && basis_error<2>() < 1e-14, "V, W and L to rounding");
 
 // (c + d J)^-1 (u, v), n = 1 / (c^2 + d^2)
 __device__ __forceinline__ void rotate(double c, double d, double n, double &u, double &v)
@@ -69,19 +107,12 @@ __device__ __forceinline__ void rotate(double c, double d, double n, double &u, 
     u = w;
 }
 
-// r (rows: eigenvectors in y, columns: in x) becomes the solution of the cell system
+// r (rows: basis in y, columns: in x) becomes the solution of the cell system
 template <int P>
 __device__ __forceinline__ void solve_modes(double sig, double tx, double ty, double (&r)[P + 1][P + 1])
 {
-    using E = Eig<P>;
+    using E = Basis<P>;
     constexpr int R = E::R;
-    if constexpr (R == 1) {
-        r[0][0] *= fast_rcp(fma(tx, E::l0, fma(ty, E::l0, sig)));
-        const double cx = fma(tx, E::a, fma(ty, E::l0, sig)), dx = tx * E::b;
-        rotate(cx, dx, fast_rcp(fma(cx, cx, dx * dx)), r[0][R], r[0][R + 1]);
-        const double cy = fma(ty, E::a, fma(tx, E::l0, sig)), dy = ty * E::b;
-        rotate(cy, dy, fast_rcp(fma(cy, cy, dy * dy)), r[R][0], r[R + 1][0]);
-    }
     const double c = fma(tx, E::a, fma(ty, E::a, sig)), dm = (tx - ty) * E::b, dp = (tx + ty) * E::b;
     double p1 = 0.5 * (r[R][R] + r[R + 1][R + 1]), p2 = 0.5 * (r[R][R + 1] - r[R + 1][R]);
     double m1 = 0.5 * (r[R][R] - r[R + 1][R + 1]), m2 = 0.5 * (r[R][R + 1] + r[R + 1][R]);
@@ -91,6 +122,20 @@ __device__ __forceinline__ void solve_modes(double sig, double tx, double ty, do
     r[R + 1][R + 1] = p1 - m1;
     r[R][R + 1] = p2 + m2;
     r[R + 1][R] = m2 - p2;
+    if constexpr (R == 1) {
+        // what the pair of an axis adds to its real eigenvalue
+#pragma unroll
+        for (int k = 1; k < 3; ++k) {
+            r[0][k] = fma(-ty, fma(E::t, r[2][k], r[1][k]), r[0][k]);
+            r[k][0] = fma(-tx, fma(E::t, r[k][2], r[k][1]), r[k][0]);
+        }
+        const double cx = fma(tx, E::a, fma(ty, E::l0, sig)), dx = tx * E::b;
+        rotate(cx, dx, fast_rcp(fma(cx, cx, dx * dx)), r[0][1], r[0][2]);
+        const double cy = fma(ty, E::a, fma(tx, E::l0, sig)), dy = ty * E::b;
+        rotate(cy, dy, fast_rcp(fma(cy, cy, dy * dy)), r[1][0], r[2][0]);
+        const double u = fma(E::t, r[2][0], r[1][0]), v = fma(E::t, r[0][2], r[0][1]);
+        r[0][0] = fma(-ty, u, fma(-tx, v, r[0][0])) * fast_rcp(fma(tx, E::l0, fma(ty, E::l0, sig)));
+    }
 }
 
 // s + c x for a constant c, without the term where c is 0
@@ -128,7 +173,7 @@ template <int P, bool SRC, bool ISO, int SX, int SY>
 __device__ __forceinline__ void sweep_rows(const SweepParams &p, int a, int g, double tx, double ty, double vol,
                                            double *ytr, double *yline)
 {
-    using E = Eig<P>;
+    using E = Basis<P>;
     constexpr int Q = P + 1, N = Q * Q, D = 3;   // D: cells in registers, the loads of two under way
     const int nx = p.nel[0], ny = p.nel[1], T = (int)blockDim.x, j = (int)threadIdx.x;
     const long long base = ((long long)g * p.Nomega + a) * p.Ndof;
