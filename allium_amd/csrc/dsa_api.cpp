@@ -81,7 +81,7 @@ constexpr int kPowerIts = 30;
 struct HostStencil {
     int dim = 0;
     int nv[3] = {1, 1, 1};
-    double h[3] = {0.0, 0.0, 0.0};   // spacing
+    double h[3] = {0.0, 0.0, 0.0};   // mean edge length along each axis of the grid
     long long N = 0;
     std::vector<double> A;  // S x N, entry (k, v) at k * N + v
     std::vector<double> dinv;
@@ -214,7 +214,22 @@ bool galerkin_dg(const allium::Mesh &m, const allium::MipMatrix &K, HostStencil 
     L.dim = dim;
     L.N = 1;
     for (int d = 0; d < 3; d++) { L.nv[d] = d < dim ? m.nel[d] + 1 : 1; L.N *= L.nv[d]; }
-    for (int d = 0; d < dim; d++) L.h[d] = std::fabs(m.h[d]);
+    for (int d = 0; d < dim; d++) {
+        // along the grid's own axis, which need not be a coordinate axis
+        const long step = d == 0 ? 1 : (d == 1 ? L.nv[0] : (long)L.nv[0] * L.nv[1]);
+        long edges = 0;
+        for (long v = 0; v < L.N; v++) {
+            if ((v / step) % L.nv[d] + 1 == L.nv[d]) continue;
+            double s2 = 0.0;
+            for (int k = 0; k < dim; k++) {
+                const double x = m.vert[(size_t)(v + step) * dim + k] - m.vert[(size_t)v * dim + k];
+                s2 += x * x;
+            }
+            L.h[d] += std::sqrt(s2);
+            edges++;
+        }
+        L.h[d] /= (double)edges;
+    }
     L.A.assign((size_t)S * L.N, 0.0);
     double scale = 0.0;
     for (long e = 0; e < m.Ne; e++)
@@ -284,7 +299,8 @@ bool coarsen(const HostStencil &F, bool all, HostStencil &C)
     C.N = 1;
     bool smaller = false;
     for (int d = 0; d < 3; d++) {
-        C.nv[d] = d < dim && (all || F.h[d] < 2.0 * hmin) ? allium::coarse_vertices(F.nv[d]) : F.nv[d];
+        // twice the closest, but for rounding, waits in every orientation of a mesh
+        C.nv[d] = d < dim && (all || F.h[d] < 1.999999 * hmin) ? allium::coarse_vertices(F.nv[d]) : F.nv[d];
         C.h[d] = F.h[d] * (C.nv[d] < F.nv[d] ? 2.0 : 1.0);
         smaller = smaller || C.nv[d] < F.nv[d];
         C.N *= C.nv[d];

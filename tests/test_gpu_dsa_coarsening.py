@@ -34,3 +34,38 @@ def test_uneven_coarsening_solves(nel, p, jitter, smooth):
     assert info["level_size"][-1] <= 729 and info["dense_coarsest"]
     # CG stops at 1e-12 of the preconditioned residual; as in test_gpu_dsa.py
     assert np.linalg.norm(x - ref) < 1e-9 * np.linalg.norm(ref)
+
+
+def _quarter_turn(v):
+    """The axes of the mesh one coordinate on: no axis lies along its own coordinate."""
+    return np.ascontiguousarray(np.stack([-v[:, 1], v[:, 0]], 1) if v.shape[1] == 2 else v[:, [2, 0, 1]])
+
+
+def _half_ring(v):
+    r, th = 1.0 + v[:, 1], np.pi * (1.0 - v[:, 0])
+    return np.ascontiguousarray(np.stack([r * np.cos(th), r * np.sin(th)], 1))
+
+
+@pytest.mark.parametrize("nel,ext,turn", [((64, 64), (1.0, 1.0), _quarter_turn), ((24, 24, 24), (1.0, 1.0, 1.0), _quarter_turn),
+                                          ((96, 24), (1.0, 2.0), _quarter_turn), ((64, 48), (1.0, 1.0), _half_ring)])
+def test_coarsening_follows_the_grid_axes(nel, ext, turn):
+    """A mesh whose axes are not coordinate axes coarsens like one with the same edges
+    along the coordinates, and needs as many CG iterations."""
+    print(f"dsa axes {nel} {turn.__name__}", flush=True)
+    ne = int(np.prod(nel))
+    rng = np.random.default_rng(3)
+    st = P.lognormal_sigma(ne, 1.0, rng) * 5
+    b = rng.normal(size=ne * 2 ** len(nel))
+    up = P.cartesian_vertices(nel, extents=ext)
+    # the ring's mean radius is 1.5: the same edge lengths on a box
+    box = P.cartesian_vertices(nel, extents=(1.5 * np.pi, 1.0)) if turn is _half_ring else up
+    got = []
+    for v in (box, turn(up)):
+        op = A.InverseAdvectionOperator(A.Mesh(nel, vertices=v), 1, 4, st)
+        dsa = A.DSA(op, 0.99 * st, cg_reltol=1e-8, cg_maxit=200)
+        dsa.solve(b)
+        got.append(dsa.info())
+    print(f"  levels {got[1]['level_size']} CG its {[g['last_cg_iterations'] for g in got]}", flush=True)
+    assert got[0]["level_size"] == got[1]["level_size"]
+    # a turned box is the same operator; the ring's cells differ by a factor 2 in width
+    assert got[1]["last_cg_iterations"] <= got[0]["last_cg_iterations"] + (0 if turn is _quarter_turn else 6)
