@@ -70,8 +70,8 @@ int export_csr(const allium::MipMatrix &K, int Ne, long long *nnz, long long *ro
 }
 
 
-// the coarsest vertex grid is inverted densely up to this size; coarsening
-// stops once a grid is at most kCoarseTarget vertices
+// the coarsest vertex grid is inverted densely up to this size; coarsening stops once
+// a grid is at most kCoarseTarget vertices, or kDenseMax if an axis would not halve evenly
 constexpr long long kDenseMax = 1331;
 constexpr long long kCoarseTarget = 729;
 // Jacobi sweeps on a coarsest grid too large for the dense inverse
@@ -144,6 +144,70 @@ bool invert(int n, double *A)
         }
     }
     std::memcpy(A, I.data(), sizeof(double) * I.size());
+    return true;
+}
+
+// Inverse of the coarsest operator: a band of bw entries on both sides of the
+// diagonal, LU with partial pivoting inside it (the pivot rows reach 2 bw to the
+// right), then the unit vectors' solutions in groups of columns, one per thread.
+// n^2 bw instead of n^3 operations of a dense inverse, and on all threads (8 of them, ms:
+// 9 x 9 x 9 vertices 170 before, 19 now, 34 x 34 590 and 26).
+bool invert_banded(int n, int bw, const std::vector<double> &M, std::vector<double> &inv)
+{
+    std::vector<double> A(M);
+    std::vector<int> piv(n);
+    auto at = [&](int r, int c) -> double & { return A[(size_t)r * n + c]; };
+    for (int c = 0; c < n; c++) {
+        const int rend = std::min(n, c + bw + 1), kend = std::min(n, c + 2 * bw + 1);
+        int p = c;
+        for (int r = c + 1; r < rend; r++)
+            if (std::fabs(at(r, c)) > std::fabs(at(p, c))) p = r;
+        if (!(std::fabs(at(p, c)) > 0)) return false;
+        piv[c] = p;
+        if (p != c)
+            for (int k = c; k < kend; k++) std::swap(at(c, k), at(p, k));
+        const double d = 1.0 / at(c, c);
+        for (int r = c + 1; r < rend; r++) {
+            const double f = at(r, c) * d;
+            at(r, c) = f;
+            if (f == 0.0) continue;
+            for (int k = c + 1; k < kend; k++) at(r, k) -= f * at(c, k);
+        }
+    }
+    inv.assign((size_t)n * n, 0.0);
+    constexpr int W = 16;   // columns of a group
+    const int groups = (n + W - 1) / W;
+    constexpr long kSplit = 4096;   // parallel_for shares a count of this size among all threads
+    allium::parallel_for(kSplit, [&](long b, long e) {
+        std::vector<double> x((size_t)n * W);
+        for (int g = (int)(groups * b / kSplit); g < (int)(groups * e / kSplit); g++) {
+            const int j0 = g * W, w = std::min(W, n - j0);
+            std::fill(x.begin(), x.end(), 0.0);
+            for (int j = 0; j < w; j++) x[(size_t)(j0 + j) * W + j] = 1.0;
+            // rows above the group's first unit vector stay zero unless a swap reaches them
+            for (int c = std::max(0, j0 - bw); c < n; c++) {
+                double *xc = &x[(size_t)c * W];
+                if (piv[c] != c) std::swap_ranges(xc, xc + W, &x[(size_t)piv[c] * W]);
+                for (int r = c + 1; r < std::min(n, c + bw + 1); r++) {
+                    const double f = A[(size_t)r * n + c];
+                    double *xr = &x[(size_t)r * W];
+                    for (int j = 0; j < W; j++) xr[j] -= f * xc[j];
+                }
+            }
+            for (int r = n - 1; r >= 0; r--) {
+                double *xr = &x[(size_t)r * W];
+                for (int k = r + 1; k < std::min(n, r + 2 * bw + 1); k++) {
+                    const double f = A[(size_t)r * n + k];
+                    const double *xk = &x[(size_t)k * W];
+                    for (int j = 0; j < W; j++) xr[j] -= f * xk[j];
+                }
+                const double d = 1.0 / A[(size_t)r * n + r];
+                for (int j = 0; j < W; j++) xr[j] *= d;
+            }
+            for (int r = 0; r < n; r++)
+                for (int j = 0; j < w; j++) inv[(size_t)r * n + j0 + j] = x[(size_t)r * W + j];
+        }
+    });
     return true;
 }
 
@@ -281,6 +345,14 @@ bool galerkin_dg(const allium::Mesh &m, const allium::MipMatrix &K, HostStencil 
         });
     }
     if (bad) { err = "vertex-space Galerkin operator is not a 3^d-point stencil"; return false; }
+    return true;
+}
+
+// an even number of elements on every axis
+bool halves_evenly(const HostStencil &F)
+{
+    for (int d = 0; d < F.dim; d++)
+        if (F.nv[d] % 2 == 0) return false;
     return true;
 }
 
@@ -820,6 +892,11 @@ int allium_dsa_create(allium_sweep_t h, const double *sigma_s, const allium_dsa_
     std::vector<HostStencil> lev(1);
     if (!galerkin_dg(m, K, lev[0], why)) return fail(ALLIUM_ERR_NUMERIC, why);
     while (lev.back().N > kCoarseTarget && lev.size() < 15) {
+        // a grid that fits the dense inverse and would not halve evenly on every axis is
+        // the coarsest: uneven halves cost CG iterations and launches (a solve on 33 x 33
+        // elements 10 iterations and 1.05 ms instead of 7 and 0.60, on 600 x 1 26 and 2.6
+        // instead of 3 and 0.30, on 9 x 10 x 11 9 and 1.02 instead of 8 and 0.74)
+        if (lev.back().N <= kDenseMax && !halves_evenly(lev.back())) break;
         HostStencil c;
         // the level count is limited: from the ninth grid on every axis is halved
         if (!coarsen(lev.back(), lev.size() > 8, c)) break;
@@ -839,17 +916,18 @@ int allium_dsa_create(allium_sweep_t h, const double *sigma_s, const allium_dsa_
     const HostStencil &Lc = lev.back();
     if (Lc.N <= kDenseMax) {
         const int Nc = (int)Lc.N, S = nstencil(Lc.dim);
-        Ainv.assign((size_t)Nc * Nc, 0.0);
+        std::vector<double> M((size_t)Nc * Nc, 0.0);
         for (int v = 0; v < Nc; v++) {
             const int c[3] = {v % Lc.nv[0], (v / Lc.nv[0]) % Lc.nv[1], v / (Lc.nv[0] * Lc.nv[1])};
             for (int k = 0; k < S; k++) {
                 const int xx = c[0] + k % 3 - 1, yy = c[1] + (k / 3) % 3 - 1, zz = c[2] + (Lc.dim > 2 ? k / 9 - 1 : 0);
                 if (xx < 0 || xx >= Lc.nv[0] || yy < 0 || yy >= Lc.nv[1] || zz < 0 || zz >= Lc.nv[2]) continue;
-                Ainv[(size_t)v * Nc + xx + Lc.nv[0] * (yy + Lc.nv[1] * zz)] += Lc.A[(size_t)k * Lc.N + v];
+                M[(size_t)v * Nc + xx + Lc.nv[0] * (yy + Lc.nv[1] * zz)] += Lc.A[(size_t)k * Lc.N + v];
             }
         }
         // row-major: each device wave reads one row
-        if (!invert(Nc, Ainv.data())) return fail(ALLIUM_ERR_NUMERIC, "DSA: singular coarsest operator");
+        const int bw = 1 + Lc.nv[0] + (Lc.dim > 2 ? Lc.nv[0] * Lc.nv[1] : 0);
+        if (!invert_banded(Nc, std::min(bw, Nc - 1), M, Ainv)) return fail(ALLIUM_ERR_NUMERIC, "DSA: singular coarsest operator");
     }
     // upload: DG blocks column-major
     auto colmajor = [&](const std::vector<double> &src, std::vector<double> &dst) { to_colmajor(n, src, dst); };

@@ -31,7 +31,8 @@ def test_uneven_coarsening_solves(nel, p, jitter, smooth):
     ref = spla.spsolve(sp.csc_matrix(K), b)
     info = dsa.info()
     print(f"  levels {info['level_size']} CG its {info['last_cg_iterations']}", flush=True)
-    assert info["level_size"][-1] <= 729 and info["dense_coarsest"]
+    # at most 729 vertices, or 1331 where an axis has an odd number of elements (9 x 10 x 11)
+    assert info["level_size"][-1] <= 1331 and info["dense_coarsest"]
     # CG stops at 1e-12 of the preconditioned residual; as in test_gpu_dsa.py
     assert np.linalg.norm(x - ref) < 1e-9 * np.linalg.norm(ref)
 
@@ -69,3 +70,20 @@ def test_coarsening_follows_the_grid_axes(nel, ext, turn):
     assert got[0]["level_size"] == got[1]["level_size"]
     # a turned box is the same operator; the ring's cells differ by a factor 2 in width
     assert got[1]["last_cg_iterations"] <= got[0]["last_cg_iterations"] + (0 if turn is _quarter_turn else 6)
+
+
+@pytest.mark.parametrize("nel,its", [((33, 33), 7), ((600, 1), 4), ((9, 10, 9), 8), ((66, 66), 13)])
+def test_small_odd_grids_keep_the_dense_inverse(nel, its):
+    """A vertex grid of 730 to 1331 vertices that does not halve evenly is the coarsest:
+    the vertex space is solved exactly and CG needs no more iterations than that allows."""
+    print(f"dsa small odd {nel}", flush=True)
+    ne = int(np.prod(nel))
+    rng = np.random.default_rng(2)
+    st = P.lognormal_sigma(ne, 1.0, rng) * 5
+    op = A.InverseAdvectionOperator(A.Mesh(nel), 1, 4, st)
+    dsa = A.DSA(op, 0.99 * st, cg_reltol=1e-8, cg_maxit=200)
+    dsa.solve(rng.normal(size=op.phi_size))
+    info = dsa.info()
+    print(f"  levels {info['level_size']} CG its {info['last_cg_iterations']}", flush=True)
+    assert 729 < info["level_size"][-1] <= 1331 and info["dense_coarsest"]
+    assert info["last_cg_iterations"] <= its + 1
