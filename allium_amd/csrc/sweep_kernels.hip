@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <mutex>
+#include <type_traits>
 
 namespace allium {
 
@@ -1274,24 +1275,25 @@ hipError_t balance_static(const SweepParams &prm, const double *psi, double *abs
 // moments (DiscreteToMoment, src/transport_op.cpp:3-46) and block mass
 // ---------------------------------------------------------------------------
 // phi = sum_a w_a psi_a: 8 + 8 / Nomega bytes per unknown, bound by HBM once
-// enough loads are in flight.  A thread that sums all directions of its entry
+// enough loads are in flight.  A thread that sums all directions of its entries
 // leaves a small phi with a few workgroups and a chain of Nomega loads each,
-// so the WV waves of a workgroup split the directions of one run of 64 E
-// entries: wave w sums its directions in order, then the waves' sums are added
-// in order through LDS (one fixed order for every launch).  psi is streamed
+// so WV waves split the directions of a run of 64 E entries: wave w sums its
+// directions in order, then the waves' sums are added in order through LDS (one
+// fixed order for every launch).  A workgroup has RW such runs.  A wave loads U
+// directions of its entries before it adds them, and what is left over by halves: with
+// few directions per wave a loop for the rest, one load at a time, took most of
+// the time (2097152 x 8 x 4 groups with 16 waves 216 us, now 99).  psi is streamed
 // once: nontemporal loads keep it from evicting the L2 and MALL lines the next
-// sweep reuses.  us for one thread per entry / this kernel: 4096 x 40 72 / 3.1,
-// 130950 x 84 130 / 16, 262144 x 80 123 / 27, 222000 x 48 x 4 groups 99 / 52,
-// 2097152 x 80 206 / 203 (6.7 TB/s).
-template <int WV, int E, int U>
-__global__ void __launch_bounds__(64 * WV) k_moments(const double *__restrict__ psi, const double *__restrict__ omega,
-                                                     int Nomega, long long Ndof, double *__restrict__ phi)
+// sweep reuses.
+template <int WV, int E, int U, int RW>
+__global__ void __launch_bounds__(64 * WV * RW) k_moments(const double *__restrict__ psi, const double *__restrict__ omega,
+                                                          int Nomega, long long Ndof, double *__restrict__ phi)
 {
-    __shared__ double part[WV][64 * E];
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
-    const long long b = (long long)blockIdx.x * (64 * E), g = blockIdx.y;
+    static_assert(WV == 1 || E <= WV, "a run's threads add its entries");
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63, w = wv % WV, r = wv / WV;
+    const long long b = ((long long)blockIdx.x * RW + r) * (64 * E), g = blockIdx.y;
     const double *ps = psi + g * Nomega * Ndof;
-    const int a0 = Nomega * w / WV, a1 = Nomega * (w + 1) / WV;
+    const int a1 = Nomega * (w + 1) / WV;
     long long i[E];
     double acc[E];
 #pragma unroll
@@ -1299,40 +1301,85 @@ __global__ void __launch_bounds__(64 * WV) k_moments(const double *__restrict__ 
         i[k] = b + l + 64 * k < Ndof ? b + l + 64 * k : Ndof - 1;
         acc[k] = 0.0;
     }
+    int a = Nomega * w / WV;
+    auto add = [&](auto count) {
+        constexpr int C = decltype(count)::value;
+        double v[C][E];
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+#pragma unroll
+            for (int k = 0; k < E; ++k) v[u][k] = __builtin_nontemporal_load(ps + (long long)(a + u) * Ndof + i[k]);
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            const double wa = omega[4 * (a + u) + 3];
+#pragma unroll
+            for (int k = 0; k < E; ++k) acc[k] = fma(wa, v[u][k], acc[k]);
+        }
+        a += C;
+    };
+    static_assert(U == 4 || U == 8, "what is left over goes by halves");
+    if constexpr (WV == 16) {
+        // at most a few directions per wave, loads and sums in the compiler's order:
+        // 2097152 x 80 201 us, 204 with the chunks
 #pragma unroll U
-    for (int a = a0; a < a1; ++a) {
-        const double wa = omega[4 * a + 3];
-        const double *pa = ps + (long long)a * Ndof;
+        for (; a < a1; ++a) {
+            const double wa = omega[4 * a + 3];
 #pragma unroll
-        for (int k = 0; k < E; ++k) acc[k] = fma(wa, __builtin_nontemporal_load(pa + i[k]), acc[k]);
+            for (int k = 0; k < E; ++k)
+                acc[k] = fma(wa, __builtin_nontemporal_load(ps + (long long)a * Ndof + i[k]), acc[k]);
+        }
+    } else {
+        while (a + U <= a1) add(std::integral_constant<int, U>{});
+        if constexpr (U == 8)
+            if (a + 4 <= a1) add(std::integral_constant<int, 4>{});
+        if (a + 2 <= a1) add(std::integral_constant<int, 2>{});
+        if (a < a1) add(std::integral_constant<int, 1>{});
     }
+    if constexpr (WV == 1) {
 #pragma unroll
-    for (int k = 0; k < E; ++k) part[w][l + 64 * k] = acc[k];
-    __syncthreads();
-    const int t = threadIdx.x;
-    if (t < 64 * E && b + t < Ndof) {
-        double s = part[0][t];
+        for (int k = 0; k < E; ++k)
+            if (b + l + 64 * k < Ndof) phi[g * Ndof + i[k]] = acc[k];
+    } else {
+        __shared__ double part[WV * RW][64 * E];
 #pragma unroll
-        for (int q = 1; q < WV; ++q) s += part[q][t];
-        phi[g * Ndof + b + t] = s;
+        for (int k = 0; k < E; ++k) part[wv][l + 64 * k] = acc[k];
+        __syncthreads();
+        const int t = (int)threadIdx.x - 64 * WV * r;
+        if (t < 64 * E && b + t < Ndof) {
+            double s = part[WV * r][t];
+#pragma unroll
+            for (int q = 1; q < WV; ++q) s += part[WV * r + q][t];
+            phi[g * Ndof + b + t] = s;
+        }
     }
+}
+
+template <int WV, int E, int U, int RW>
+static hipError_t launch_moments_t(const SweepParams &prm, const double *psi, double *phi, hipStream_t s)
+{
+    constexpr int run = 64 * E * RW;
+    hipLaunchKernelGGL((k_moments<WV, E, U, RW>), dim3((unsigned)((prm.Ndof + run - 1) / run), (unsigned)prm.G),
+                       dim3(64 * WV * RW), 0, s, psi, prm.omega, prm.Nomega, prm.Ndof, phi);
+    return hipGetLastError();
 }
 
 hipError_t launch_moments(const SweepParams &prm, const double *psi, double *phi, hipStream_t s)
 {
-    // A psi that outgrows the 256 MB MALL is read from HBM: 16 waves of a
-    // workgroup on 1 KB runs reach 6.7 TB/s (203 us at 2097152 x 80, against
-    // 216 with 4 waves on 512 B).  Below, psi is partly in the MALL and more,
-    // smaller workgroups are faster: 262144 x 80 (168 MB) 27 against 36 us,
-    // 222000 x 48 x 4 (341 MB) 52 against 58.
-    const double bytes = 8.0 * prm.Ndof * prm.Nomega * prm.G;
-    if (bytes > 5e8)
-        hipLaunchKernelGGL((k_moments<16, 2, 4>), dim3((unsigned)((prm.Ndof + 127) / 128), (unsigned)prm.G),
-                           dim3(1024), 0, s, psi, prm.omega, prm.Nomega, prm.Ndof, phi);
-    else
-        hipLaunchKernelGGL((k_moments<4, 1, 8>), dim3((unsigned)((prm.Ndof + 63) / 64), (unsigned)prm.G), dim3(256),
-                           0, s, psi, prm.omega, prm.Nomega, prm.Ndof, phi);
-    return hipGetLastError();
+    // Splitting the directions needs enough of them, and its runs of 512 B enough rows on
+    // 64-byte boundaries.  us of <1,4,4,4> / <4,1,8,1> / <4,2,4,1> / <16,2,4,1> at
+    // entries x directions x groups:
+    //   few directions, many entries: 2097152 x 8 24 / 25 / 28 / 52, 2000001 x 12 x 2 71 / 83 / 73 / 105
+    //   few directions, few entries: 262144 x 8 4.6 / 4.5 / 3.1 / 5.7, 22500 x 12 5.4 / 2.7 / 2.7 / 2.7
+    //   rows off 64 bytes, many entries: 1771561 x 24 57 / 67 / 62 / 69, 300763 x 80 x 4 123 / 155 / 138 / 137
+    //   others: 262144 x 24 x 16 137 / 136 / 151 / 184, 262144 x 80 30 / 26 / 33 / 36
+    //   many directions, psi over 1 GB: 2097152 x 80 221 / 212 / 216 / 201 (6.7 TB/s); smaller: 1500000 x
+    //   80 148 / 149 / 151 / 146, 512000 x 80 x 2 99 / 101 / 106 / 105
+    const double entries = (double)prm.Ndof * prm.G, bytes = 8.0 * entries * prm.Nomega;
+    const bool many = entries >= 524288.0;
+    if (many && (prm.Nomega < 16 || prm.Ndof % 8)) return launch_moments_t<1, 4, 4, 4>(prm, psi, phi, s);
+    if (prm.Nomega < 16) return launch_moments_t<4, 2, 4, 1>(prm, psi, phi, s);
+    if (prm.Nomega >= 64 && bytes > 1e9) return launch_moments_t<16, 2, 4, 1>(prm, psi, phi, s);
+    return launch_moments_t<4, 1, 8, 1>(prm, psi, phi, s);
 }
 
 // [phi, J_0, .., J_{dim-1}] with the moment index slowest: mom[(m G + g) Ndof + s]

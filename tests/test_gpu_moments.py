@@ -24,3 +24,14 @@ def test_moments_match_the_sum(nel, p, sn, G):
     # each partial sum is rounded once per direction and once per wave
     bound = (op.Nomega + 16) * 2.0 ** -52 * np.einsum("a,gai->gi", w, np.abs(ps)).reshape(-1)
     assert (np.abs(phi - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("nel,p,sn,G", [((121, 61, 72), 0, 2, 1),       # few directions, many entries
+                                        ((263, 251), 0, 4, 9),          # and several groups, rows off 64 bytes
+                                        ((13, 7), 0, 4, 2),             # few directions, few entries
+                                        ((81, 83, 79), 0, 4, 1),        # 24 directions, rows off 64 bytes
+                                        ((5, 5, 5), 0, 6, 4),           # the same with few entries
+                                        ((17, 9, 5), 1, 6, 2),          # 12 directions per wave: a chunk of 8 and one of 4
+                                        ((58, 59, 58), 1, 8, 1)])       # over 1 GB
+def test_moments_of_every_split(nel, p, sn, G):
+    test_moments_match_the_sum(nel, p, sn, G)
