@@ -955,8 +955,12 @@ __global__ void __launch_bounds__(256) k_apply_L(SweepParams p, const double *__
     const long long item = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long total = (long long)p.Ne * p.Nomega * p.G;
     if (item >= total) return;
-    const int e = (int)(item % p.Ne);
-    const int a = (int)((item / p.Ne) % p.Nomega);
+    // A wave's lanes share what is large: K of their direction on uniform geometry, the
+    // matrices of their element on general geometry.  (With the elements innermost
+    // there too every direction read all matrices again, each lane its own: 24^3 p = 2
+    // S8 26 ms, now 3.8, 8 x 9 x 10 p = 2 S8 0.88 and 0.29, 26 x 23 x 29 p = 1 S8 3.4 and 0.31.)
+    const int first = UNI ? p.Ne : p.Nomega, lo = (int)(item % first), hi = (int)((item / first) % (UNI ? p.Nomega : p.Ne));
+    const int e = UNI ? lo : hi, a = UNI ? hi : lo;
     const int g = (int)(item / ((long long)p.Ne * p.Nomega));
     int c[3] = {e % p.nel[0], (e / p.nel[0]) % p.nel[1], e / (p.nel[0] * p.nel[1])};
     const double om[3] = {p.omega[4 * a], p.omega[4 * a + 1], p.omega[4 * a + 2]};
@@ -978,11 +982,15 @@ __global__ void __launch_bounds__(256) k_apply_L(SweepParams p, const double *__
     } else {
 #pragma unroll
         for (int i = 0; i < N; ++i) yl[i] = 0.0;
-        // column by column, as the gradient blocks are stored (the masses are symmetric)
+        // Column by column, as the gradient blocks are stored (the masses are symmetric).
+        // At 3D p = 2 the columns are a loop: unrolled, their 2916 loads fill the instruction
+        // cache (4^3 S8 208 us instead of 189, 24^3 S8 4.1 ms instead of 3.8).
         const double *Gd = p.Gd + (size_t)e * DIM * N * N, *Mu = p.Mu + (size_t)e * N * N;
         const double *Mt = p.Mt + (size_t)e * N * N;
-#pragma unroll
-        for (int j = 0; j < N; ++j)
+        constexpr int UJ = N > 9 ? 1 : N;
+#pragma unroll UJ
+        for (int j = 0; j < N; ++j) {
+            const double xj = UJ == 1 ? xe[j] : xl[j];
 #pragma unroll
             for (int i = 0; i < N; ++i) {
                 double v = om[0] * Gd[j * N + i];
@@ -990,8 +998,9 @@ __global__ void __launch_bounds__(256) k_apply_L(SweepParams p, const double *__
                 for (int d = 1; d < DIM; ++d) v = fma(om[d], Gd[(d * N + j) * N + i], v);
                 v = fma(sig, Mu[j * N + i], v);
                 if (p.timedep) v = fma(p.tau, Mt[j * N + i], v);
-                yl[i] = fma(v, xl[j], yl[i]);
+                yl[i] = fma(v, xj, yl[i]);
             }
+        }
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
