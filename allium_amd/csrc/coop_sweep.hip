@@ -335,9 +335,9 @@ __device__ __forceinline__ void coop_wave(const SweepParams &p, const CoopLevel 
         auto uv = [&](int v) { return v == 0 ? lo : (v == P ? hi : zero); };
         // Columns in node order, CH at a time: the loads of the next chunk are issued
         // before the products of this one (NB = 2 buffers).  At p = 1 all columns fit.
-        // A p = 2 uniform mesh reads fewer lines and is faster with one column at a
-        // time and a third wave in the registers (24^3 S12: 4.5 against 5.5 ms).
-        constexpr int CH = P == 1 ? N : (UNI ? 1 : Q), NC = N / CH, NB = NC > 1 && !UNI ? 2 : 1;
+        // (One column at a time, for a third wave in the registers, is slower on uniform
+        // meshes too: 24^3 S12 4.76 ms against 4.24, 3^3 S4 106 us against 81.)
+        constexpr int CH = P == 1 ? N : Q, NC = N / CH, NB = NC > 1 ? 2 : 1;
         static_assert(N % CH == 0, "whole chunks");
         double u[NB][CH], m[NB][CH][RS], f[NB][CH][RS];
         auto load = [&](auto cc) {
@@ -360,7 +360,6 @@ __device__ __forceinline__ void coop_wave(const SweepParams &p, const CoopLevel 
         for_each_k(
             [&](auto cc) {
                 constexpr int c = decltype(cc)::value, v = c % NB;
-                if constexpr (UNI) asm volatile("" : "+v"(mat), "+v"(fb), "+v"(lo), "+v"(hi), "+v"(b[0]));
                 load(std::integral_constant<int, c + NB - 1>{});
 #pragma unroll
                 for (int i = 0; i < CH; ++i) {
@@ -464,7 +463,7 @@ __device__ __forceinline__ void coop_wave(const SweepParams &p, const CoopLevel 
 // instantiations so that the parameters' address space is known (a pointer
 // selected between the two would be generic and its loads flat).
 template <int P, bool UNI, typename T, bool BATCH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P == 1 ? 4 : (UNI ? 3 : 2))))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P == 1 ? 4 : 2)))
 k_sweep_coop(SweepParams p0, const SweepParams *__restrict__ prms, CoopLevel cl)
 {
     // Workgroups go to the 8 XCDs round robin (blockIdx.x % 8).  Each XCD takes
