@@ -771,17 +771,18 @@ int allium_sweep_set_launch(allium_sweep_t h, int mode)
     struct Cand { int mode, block, lanes, bx, by, bz, nd, pf; };
     std::vector<Cand> cands;
     const bool coop = allium::coop_supported(h->mesh.dim, h->ed.p);
-    if (coop) {
+    // cooperative level launches have one workgroup size and one number of lanes
+    const bool coop_levels = allium::coop_level_supported(h->mesh.dim, h->ed.p, h->mesh.uniform);
+    if (coop_levels) {
         cands.push_back({0, 256, 1, 0, 0, 0, 0, 0});
         cands.push_back({1, 256, 1, 0, 0, 0, 0, 0});
     }
-    if (coop) {
-    } else if (h->ds.angle_independent)
+    if (!coop && h->ds.angle_independent)
         for (int bl : {256, 512}) cands.push_back({3, bl, 1, 0, 0, 0, 0, 0});
     for (int md : {0, 1})
         for (int bl : {64, 128, 256})
             for (int ln : {0, 1, 2, 4}) {
-                if (coop) continue;
+                if (coop_levels) continue;
                 if (ln == 0 && !h->ds.d_wcells) continue;
                 if (ln > 0 && h->ed.n % ln) continue;
                 cands.push_back({md, bl, ln, 0, 0, 0, 0, 0});

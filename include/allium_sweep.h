@@ -108,9 +108,10 @@ int allium_sweep_set_precision(allium_sweep_t h, int precision);
 int allium_sweep_set_launch(allium_sweep_t h, int mode);
 /* explicit tuning: launch mode, workgroup size (64..256, multiple of 64; up
  * to 512 for mode 3, 1024 for box sweeps at p = 1) and
- * lanes per cell (1, 2 or 4: each lane owns n/lanes rows of a cell's system,
- * without effect at 3D p = 1 on general geometry, where 8 lanes solve a cell;
- * 0: one lane per cell in direction-uniform waves over XCD-local spatial bins,
+ * lanes per cell (1, 2 or 4: each lane owns n/lanes rows of a cell's system;
+ * size and lanes are without effect on level launches at 3D p = 2 and at 3D p = 1 on
+ * general geometry, where 256 threads take 16 or 8 lanes per cell, and the autotuner
+ * tries and reports 256 and 1 there; 0: one lane per cell in direction-uniform waves over XCD-local spatial bins,
  * uniform geometry only; modes 3..5 take 1) */
 int allium_sweep_set_tuning(allium_sweep_t h, int mode, int block, int lanes);
 int allium_sweep_get_tuning(allium_sweep_t h, int *mode, int *block, int *lanes);

@@ -42,3 +42,17 @@ def test_matches_oracle(nel, p, sn, G, jitter, tau):
     op.Mult(A.DeviceVector.from_host(q), psi)
     # 24-bit factors of well conditioned systems of up to 27 unknowns, a few cells deep
     assert rel_err(psi.to_host(), ref) < 1e-4
+
+
+def test_autotuner_tries_cooperative_levels_once():
+    """Level launches on 3D p = 1 general geometry have one workgroup size and one number of
+    lanes: the tuner reports these, not what the last timings happened to favour."""
+    nel = (3, 4, 5)
+    v = P.jittered_vertices(nel, 0.05, np.random.default_rng(2))
+    op = A.InverseAdvectionOperator(A.Mesh(nel, vertices=v), 1, 4, np.ones((8, 60)))
+    op.set_tuning(0, 64, 4)
+    for _ in range(3):
+        op.set_launch(-1)
+        t = op.tuning()
+        assert t["mode"] in (0, 1, 3) and t["lanes"] == 1
+        assert t["mode"] == 3 or t["block"] == 256
