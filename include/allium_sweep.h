@@ -94,7 +94,9 @@ int allium_sweep_get_time_absorption(allium_sweep_t h, double *tau);
 int allium_sweep_get_lumping(allium_sweep_t h, int *lump, int *parallel_block_jacobi);
 /* ALLIUM_FP64 or ALLIUM_FP32_REFINED local solves: the latter assembles and
  * factors each cell's system in FP32 (FP64 vectors in and out); FP64 accuracy
- * is restored by the defect correction of allium_source_iteration */
+ * is restored by the defect correction of allium_source_iteration.  Where FP32
+ * cells are not faster the request is served by the FP64 ones: 3D p = 2 on uniform
+ * geometry, and 2D p = 1, 2 on uniform geometry in mode 3 (unlumped) */
 int allium_sweep_set_precision(allium_sweep_t h, int precision);
 /* 0 = one launch per level, 1 = hipGraph of level launches, 2 = persistent
  * kernel with device-side level counters (disabled), 3 = one workgroup per

@@ -116,3 +116,63 @@ def test_rows_are_accurate(nel, log_sd, p):
     # A basis of condition 7 per axis (p = 2) gave 5 to 13 times the LU's error, constants
     # that err by 3e-16 in every element (p = 1) 5 to 10 times on the larger meshes.
     assert err[3] < (5.0 if p == 1 else 2.5) * err[0]
+
+
+@pytest.mark.parametrize("nel,p", [((9, 70), 1), ((9, 70), 2), ((3, 4, 5), 2)])
+def test_fp32_requests_that_run_fp64(nel, p):
+    """2D rows and uniform 3D p = 2 cells serve FP32 requests in FP64, to the bit."""
+    op = A.InverseAdvectionOperator(A.Mesh(nel), p, 4, np.ones((1, int(np.prod(nel)))))
+    op.set_launch(3 if len(nel) == 2 else 0)
+    q = A.DeviceVector.from_host(np.random.default_rng(1).uniform(0.1, 1.0, op.size))
+    psi = [op.Mult(q, A.DeviceVector(op.size)).to_host()]
+    op.set_precision(A.FP32_REFINED)
+    psi.append(op.Mult(q, A.DeviceVector(op.size)).to_host())
+    np.testing.assert_array_equal(*psi)
+
+
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("nel,block", [((9, 5), 64), ((6, 150), 64)])
+def test_rows_with_both_sources(nel, block, p):
+    """A source per direction and an isotropic one together, as source iteration has them."""
+    rng = np.random.default_rng(9)
+    ne = int(np.prod(nel))
+    sig = P.lognormal_sigma(2 * ne, 1.0, rng).reshape(2, ne)
+    v = P.cartesian_vertices(nel, extents=(2.0, 1.0))
+    op = A.InverseAdvectionOperator(A.Mesh(nel, vertices=v), p, 6, sig)
+    op.set_tuning(3, block, 1)
+    om, w = ls_fixture(6, 2)
+    pr = oracle.Problem(2, nel, v, p, om, w, sig)
+    q, iso = rng.uniform(0.1, 1.0, op.size), rng.uniform(0.1, 1.0, op.phi_size)
+    ref = np.empty(op.size)
+    pr.sweep(q + np.broadcast_to(iso.reshape(2, 1, -1), (2, op.Nomega, op.phi_size // 2)).reshape(-1), ref)
+    psi, phi = A.DeviceVector.from_host(np.full(op.size, np.nan)), A.DeviceVector(op.phi_size)
+    op.MultMoments(A.DeviceVector.from_host(q), psi, phi, A.DeviceVector.from_host(iso))
+    # FP64 both, in other elimination orders; the moments sum positive terms
+    assert rel_err(psi.to_host(), ref) < 1e-12
+    assert rel_err(phi.to_host(), np.einsum("a,gai->gi", w, ref.reshape(2, op.Nomega, -1)).reshape(-1)) < 1e-12
+
+
+# the traces of a strip's last row take 8 Q nx bytes of LDS next to 16 Q block of the lanes:
+# 64 KB are 3968 elements at p = 1 and 2602 at p = 2 with 64 lanes
+@pytest.mark.parametrize("nel,p,lump", [((3968, 65), 1, 0), ((3969, 65), 1, 0), ((2602, 65), 2, 0), ((2603, 65), 2, 0),
+                                        ((12, 70), 1, 7), ((12, 70), 1, 1)])
+def test_direction_sweeps_where_rows_stop(nel, p, lump):
+    """Both sides of the LDS bound, and lumped matrices, which the rows do not take."""
+    print(f"rows bound {nel} p={p} lump {lump}", flush=True)
+    rng = np.random.default_rng(10)
+    ne = int(np.prod(nel))
+    sig = P.lognormal_sigma(ne, 1.0, rng).reshape(1, -1) * nel[0]
+    # one direction per quadrant keeps the oracle short
+    om = np.array([[0.7, 0.3], [-0.7, 0.3], [0.3, -0.7], [-0.3, -0.7]])
+    w = np.full(4, 0.25)
+    v = P.cartesian_vertices(nel)
+    op = A.InverseAdvectionOperator(A.Mesh(nel, vertices=v), p, (om, w), sig, lump=lump)
+    op.set_tuning(3, 64, 1)
+    pr = oracle.Problem(2, nel, v, p, om, w, sig, lump=lump)
+    q = rng.uniform(0.1, 1.0, op.size)
+    ref = np.empty(op.size)
+    pr.sweep(q, ref)
+    psi = A.DeviceVector.from_host(np.full(op.size, np.nan))
+    op.Mult(A.DeviceVector.from_host(q), psi)
+    # relative to the largest value: FP64 both, in other elimination orders
+    assert rel_err(psi.to_host(), ref) < 1e-12
