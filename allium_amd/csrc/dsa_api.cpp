@@ -235,7 +235,7 @@ void host_mv(const allium::MipMatrix &K, int Ne, const double *x, double *y)
 void host_st_mv(const HostStencil &L, const double *x, double *y)
 {
     const int S = nstencil(L.dim);
-    allium::parallel_for(L.N, [&](long b, long vend) {
+    auto rows = [&](long b, long vend) {
         for (long v = b; v < vend; v++) {
             const int c[3] = {(int)(v % L.nv[0]), (int)((v / L.nv[0]) % L.nv[1]), (int)(v / ((long)L.nv[0] * L.nv[1]))};
             double acc = 0.0;
@@ -246,7 +246,10 @@ void host_st_mv(const HostStencil &L, const double *x, double *y)
             }
             y[v] = acc;
         }
-    });
+    };
+    // starting threads takes about 0.3 ms, a product on 16384 vertices 0.1 to 0.4 ms
+    if (L.N < 16384) rows(0, L.N);
+    else allium::parallel_for(L.N, rows);
 }
 
 // largest eigenvalue of D^{-1} A by power iteration (D^{-1} A is similar to a
