@@ -25,9 +25,10 @@
 // element with the other cells' coefficients zero.  Reading each row per cell
 // (27 doubles 216 B apart in every lane) kept the L1's return path busy 94 % of
 // the time.  Measured before / after, ms: 16^3 + 18^3 + 21^3 p = 2 S12 batch 10.7 / 8.2,
-// uniform 24^3 p = 2 S12 5.1 / 4.6, 26 x 23 x 29 p = 1 S8 (one lane per cell before)
-// 1.80 / 0.90, 48^3 p = 1 S8 8.2 / 3.2.  What is left is issue: about 2000 vector and
-// 216 matrix instructions per wave of four 27 x 27 cells at two waves per SIMD.
+// uniform 24^3 p = 2 S12 5.3 / 4.2, 26 x 23 x 29 p = 1 S8 (one lane per cell before)
+// 1.80 / 0.90, 48^3 p = 1 S8 8.2 / 3.2.  What is left is issue: 2000 to 2300 vector and
+// 162 matrix instructions (a few more where a wave holds several elements) per wave of
+// four 27 x 27 cells, counted, at two waves per SIMD.
 #include <type_traits>
 #include <utility>
 
@@ -491,8 +492,8 @@ hipError_t launch_pu(const SweepParams &p0, const SweepParams *d_prms, const Coo
     constexpr int per = 4 * Coop<P>::CPW;
     static_assert(P != 2 || per == kCoopCells, "instances start on a workgroup");
     const dim3 grid((unsigned)((items + per - 1) / per)), block(256);
-    // FP32 solves of uniform p = 2 cells save nothing (24^3 S12: 4.72 ms against 4.57
-    // in FP64): they are the FP64 ones
+    // FP32 solves of uniform p = 2 cells saved nothing (24^3 S12: 4.72 ms against 4.57
+    // in FP64, with one column at a time): they are the FP64 ones
     constexpr bool f32 = !(P == 2 && UNI);
     using F = std::conditional_t<f32, float, double>;
     if constexpr (P == 2) {

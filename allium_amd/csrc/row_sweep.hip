@@ -28,11 +28,11 @@
 // (condition 7 per axis) needs 12 instructions fewer and was at 1.5e-14.  At p = 1 3.7e-15
 // (LU 2.6e-15, box sweeps 2.0e-14): the pair's unknowns are three times their trace.
 //
-// Bound by issue: about 330 (p = 2) and 150 (p = 1) instructions a step in each of a
-// few waves per CU, one per about 8 cycles.  A 9 x 9 LU in one lane with the traces
-// read back from memory took 3 us a step.  Measured before / after (the best launch
-// mode of each), us: 150 x 97 p = 2 S12 728 / 186, 300 x 300 p = 2 S12 2608 / 1200,
-// 150 x 97 p = 1 S12 271 / 102, 32 x 32 p = 1 S8 45 / 30.
+// Bound by issue: about 350 (p = 2) and 170 (p = 1) instructions a step in each of a few
+// waves per CU, 230 and 101 of them vector ones, one of those per 8 cycles.  A 9 x 9 LU in
+// one lane with the traces read back from memory took 3 us a step.  Measured before / after
+// (the best launch mode of each, one pair of vectors), us: 150 x 97 p = 2 S12 728 / 187, 300 x
+// 300 p = 2 S12 2608 / 1178, 150 x 97 p = 1 S12 271 / 102, 32 x 32 p = 1 S8 45 / 30.
 #include <algorithm>
 
 #include "device.hpp"

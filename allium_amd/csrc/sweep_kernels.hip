@@ -801,7 +801,7 @@ template <int DIM, int P, bool UNI, typename T>
 static hipError_t run_directions(DeviceSweep &ds, const SweepParams &prm, hipStream_t stream)
 {
     // 2D boxes by rows of elements, FP64 cells at either precision: 150 x 97 p = 2 S12
-    // 186 us, 728 with one lane per cell and an LU
+    // 187 us, 728 with one lane per cell and an LU (on one pair of vectors)
     if (DIM == 2 && UNI && row_sweep_block(ds)) return launch_row_sweep(ds, prm, stream);
     const int block = std::max(64, std::min(512, ds.dir_block));
     hipLaunchKernelGGL((k_sweep_direction<DIM, P, UNI, T>), dim3(prm.Nomega, prm.G), dim3(block), 0, stream, prm,
@@ -815,7 +815,8 @@ static hipError_t run_mode(DeviceSweep &ds, const SweepParams &prm, hipStream_t 
     if (mode == 3) return run_directions<DIM, P, UNI, T>(ds, prm, stream);
     if (mode == 2) return run_persistent<DIM, P, UNI, T>(ds, prm, stream);
     // 3D p = 1 on general geometry: cooperative cells whatever ds.lanes (26 x 23 x 29
-    // S8: 0.77 ms against 1.68 with the best of 1, 2 and 4 lanes of own rows)
+    // S8, one pair of vectors: 0.77 ms against 1.68 with the best of 1, 2 and 4 lanes of
+    // own rows)
     if constexpr (DIM == 3 && P == 1 && !UNI) return run_coop(ds, prm, stream, mode);
     else return run_levels<DIM, P, UNI, T>(ds, prm, stream);
 }
