@@ -771,12 +771,12 @@ int allium_sweep_set_launch(allium_sweep_t h, int mode)
     struct Cand { int mode, block, lanes, bx, by, bz, nd, pf; };
     std::vector<Cand> cands;
     const bool coop = allium::coop_supported(h->mesh.dim, h->ed.p);
-    // cooperative level launches have one workgroup size and one number of lanes
+    // Cooperative level launches have one workgroup size and one number of lanes.  Plain
+    // launches and their graph are within a percent of each other: the best of three.
     const bool coop_levels = allium::coop_level_supported(h->mesh.dim, h->ed.p, h->mesh.uniform);
-    if (coop_levels) {
-        cands.push_back({0, 256, 1, 0, 0, 0, 0, 0});
-        cands.push_back({1, 256, 1, 0, 0, 0, 0, 0});
-    }
+    if (coop_levels)
+        for (int rep = 0; rep < 3; rep++)
+            for (int md : {0, 1}) cands.push_back({md, 256, 1, 0, 0, 0, 0, 0});
     if (!coop && h->ds.angle_independent)
         for (int bl : {256, 512}) cands.push_back({3, bl, 1, 0, 0, 0, 0, 0});
     for (int md : {0, 1})

@@ -176,3 +176,21 @@ def test_direction_sweeps_where_rows_stop(nel, p, lump):
     op.Mult(A.DeviceVector.from_host(q), psi)
     # relative to the largest value: FP64 both, in other elimination orders
     assert rel_err(psi.to_host(), ref) < 1e-12
+
+
+@pytest.mark.parametrize("p", [1, 2])
+def test_rows_along_the_axes(p):
+    """Directions along an axis: one of t_x, t_y is zero."""
+    nel, ne = (7, 66), 7 * 66
+    sig = P.lognormal_sigma(ne, 1.0, np.random.default_rng(11)).reshape(1, -1)
+    om = np.array([[1.0, 0.0], [-1.0, 0.0], [0.0, 1.0], [0.0, -1.0]])
+    w = np.full(4, 0.25)
+    op = A.InverseAdvectionOperator(A.Mesh(nel), p, (om, w), sig)
+    op.set_tuning(3, 64, 1)
+    pr = oracle.Problem(2, nel, P.cartesian_vertices(nel), p, om, w, sig)
+    q = np.random.default_rng(12).uniform(0.1, 1.0, op.size)
+    ref = np.empty(op.size)
+    pr.sweep(q, ref)
+    psi = op.Mult(A.DeviceVector.from_host(q), A.DeviceVector.from_host(np.full(op.size, np.nan)))
+    # FP64 both, in other elimination orders
+    assert rel_err(psi.to_host(), ref) < 1e-12
