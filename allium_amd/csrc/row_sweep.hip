@@ -18,15 +18,16 @@
 // of both axes the system is solved from the pair (x) pair unknowns (two 2 x 2
 // rotations in the +- eigenspaces of the product of the two axes' J = [[0, 1], [-1, 0]])
 // over pair (x) real (a rotation each) to real (x) real.  V is orthogonal under m but for
-// the ratio of the pair's two scales (1.9 at p = 1, 1.7 at p = 2).  The traces are passed
+// the scales of its columns and a ratio of the pair's two scales (1.9 at p = 1, 1.7 at p = 2).  The traces are passed
 // on in the basis of their own axis, so a step's chain from trace to trace is 2 Q^2
 // multiply-adds, the solve, and a few additions; the transform of the source, the
 // reciprocals and the transform to nodal values hang off it.
 //
-// Error (2-norm against extended precision, log-normal sigma): that of the LU within a
-// third at p = 2 (2.3e-15 on 150 x 97, LU 2.9e-15); a basis of eigenvectors
-// (condition 7 per axis) needs 12 instructions fewer and was at 1.5e-14.  At p = 1 3.7e-15
-// (LU 2.6e-15, box sweeps 2.0e-14): the pair's unknowns are three times their trace.
+// Error (2-norm against extended precision): at p = 2 that of the LU (log-normal sigma, 150
+// x 97: 2.3e-15, LU 2.9e-15) to twice it (constant sigma, 61 x 47: 4.6e-15, LU 2.2e-15); a
+// basis of eigenvectors (condition 7 per axis) needs 12 instructions fewer and was at
+// 1.5e-14 on the first.  At p = 1 3.7e-15 there (LU 2.6e-15, box sweeps 2.0e-14): the pair's
+// unknowns are three times their trace.
 //
 // Bound by issue: about 350 (p = 2) and 170 (p = 1) instructions a step in each of a few
 // waves per CU, 230 and 101 of them vector ones, one of those per 8 cycles.  A 9 x 9 LU in
